@@ -211,8 +211,15 @@ int lbm_run(const lbm_step_args* args, int64_t nsteps, void* stream);
  * split post-streaming run), contiguous extent a multiple of 64, i1 extent a
  * multiple of 8; by default for D3Q19 in every storage format and for D3Q27
  * in FP32), plan[1] = single-step launches.  No lettuce counterpart; for
- * reporting. */
+ * reporting.  On 2D grids lbm_run may take the pull steps of this plan
+ * several per launch instead: lbm_run_launches counts the launches made. */
 int lbm_run_plan(const lbm_step_args* args, int64_t nsteps, int64_t* plan);
+
+/* The launches lbm_run makes for `nsteps` steps, without launching anything:
+ * launches[0] of the several-step kernel for 2D grids (D2Q9, any extents,
+ * with or without boundaries, up to 10 steps each), launches[1] of the
+ * two-step kernels, launches[2] of single steps.  For reporting. */
+int lbm_run_launches(const lbm_step_args* args, int64_t nsteps, int64_t* launches);
 
 /* Launch tuning for measurements and tests (no lettuce counterpart): set the
  * process-wide knob `name` to `value`, or back to the value its environment
@@ -220,8 +227,11 @@ int lbm_run_plan(const lbm_step_args* args, int64_t nsteps, int64_t* plan);
  * default selection, 2 wherever the two-step kernel applies),
  * "two_step_planes" (x chunk, 0 = per grid), "two_step_barriers" (1 or 2,
  * 0 = per format), "wide_offsets" (1 forces 64-bit plane offsets),
- * "post_split" (0 runs post-streaming with the push kernel only).  Not
- * synchronised with launches on other threads. */
+ * "post_split" (0 runs post-streaming with the push kernel only),
+ * "multi_step" (the several-step kernel for 2D grids: 0 never, 1 default
+ * selection, 2 wherever it applies; "two_step" 0 turns it off too),
+ * "multi_step_depth", "multi_step_tile1", "multi_step_tile2" (most steps per
+ * launch and the tile's extents, 0 = per grid).  Not synchronised with launches on other threads. */
 int lbm_set_tuning(const char* name, int32_t value);
 
 /* f[q][cell] = feq_q(rho[cell], u[:, cell]) written in the given storage:

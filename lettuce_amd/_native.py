@@ -95,6 +95,7 @@ _SIGNATURES = {
                         _vp], ctypes.c_int),
     "lbm_enstrophy_f64": ([_i32, _I64_3, _vp, _vp, _vp, _vp], ctypes.c_int),
     "lbm_run_plan": ([ctypes.POINTER(LbmStepArgs), _i64, _vp], ctypes.c_int),
+    "lbm_run_launches": ([ctypes.POINTER(LbmStepArgs), _i64, _vp], ctypes.c_int),
     "lbm_scan_f64": ([_i32, _i32, _I64_3, _I64_4, _vp, _dbl, _vp, _vp, _vp], ctypes.c_int),
     "lbm_link_force_f64": ([_i32, _i32, _I64_3, _I64_4, _vp, _dbl, _vp, _i64,
                             _vp, _vp, _vp], ctypes.c_int),
@@ -160,7 +161,8 @@ def check(rc, what):
 class tuning:
     """Context manager that sets launch-tuning knobs of the library
     (lbm_set_tuning: two_step, two_step_planes, two_step_barriers,
-    wide_offsets, post_split) and restores their start values on exit.
+    wide_offsets, post_split, multi_step, multi_step_depth, multi_step_tile1,
+    multi_step_tile2) and restores their start values on exit.
     The knobs are process-wide; they exist for measurements and tests."""
 
     def __init__(self, **knobs):

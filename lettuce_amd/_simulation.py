@@ -155,12 +155,21 @@ class NativeStep:
             self.flow.swap()
 
     def plan(self, nsteps: int):
-        """(two-step launches, single-step launches) that run(nsteps) makes"""
+        """(two-step launches, single-step launches) that run(nsteps) splits
+        into where no launch takes more than two steps (see launches)"""
         self._bind_buffers()
         out = (ctypes.c_int64 * 2)()
         N.check(N.lib().lbm_run_plan(ctypes.byref(self.args), int(nsteps), out),
                 "lbm_run_plan")
         return int(out[0]), int(out[1])
+
+    def launches(self, nsteps: int):
+        """(several-step, two-step, single-step) launches that run(nsteps) makes"""
+        self._bind_buffers()
+        out = (ctypes.c_int64 * 3)()
+        N.check(N.lib().lbm_run_launches(ctypes.byref(self.args), int(nsteps), out),
+                "lbm_run_launches")
+        return tuple(int(k) for k in out)
 
 
 class Simulation:

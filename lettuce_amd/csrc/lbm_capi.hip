@@ -16,6 +16,7 @@
 #include "lbm_step_impl.h"
 #include "lbm_slab.h"
 #include "lbm_tb2.h"
+#include "lbm_tile2d.h"
 
 namespace lbm {
 KernelFn pick_kernel_d2q9(int storage, int coll, bool mask, int mode);
@@ -39,6 +40,12 @@ int launch_learned(const KParams& p, const lbm_learned* l, int stencil, int stor
 //                                               offsets (0: chosen per grid)
 //  post_split         LETTUCE_AMD_POST_SPLIT    0 runs post-streaming with the
 //                                               push kernel only (see lbm_run)
+//  multi_step         LETTUCE_AMD_MULTI         0 never, 1 the default
+//                                               selection (see tile2d_choice),
+//                                               2 wherever it applies
+//  multi_step_depth   LETTUCE_AMD_MULTI_DEPTH   most steps per launch
+//  multi_step_tile1   LETTUCE_AMD_MULTI_TILE1   tile extents along i1 and i2
+//  multi_step_tile2   LETTUCE_AMD_MULTI_TILE2   (all three: 0 chosen per grid)
 namespace {
 struct Knob {
   const char* name;
@@ -53,8 +60,13 @@ Knob g_knobs[] = {
     {"two_step_barriers", "LETTUCE_AMD_TB2_BARRIERS", 0, 0, 0},
     {"wide_offsets", "LETTUCE_AMD_WIDE", 0, 0, 0},
     {"post_split", "LETTUCE_AMD_POST_SPLIT", 1, 0, 0},
+    {"multi_step", "LETTUCE_AMD_MULTI", 1, 0, 0},
+    {"multi_step_depth", "LETTUCE_AMD_MULTI_DEPTH", 0, 0, 0},
+    {"multi_step_tile1", "LETTUCE_AMD_MULTI_TILE1", 0, 0, 0},
+    {"multi_step_tile2", "LETTUCE_AMD_MULTI_TILE2", 0, 0, 0},
 };
-enum KnobId { K_TWO_STEP, K_TB2_PLANES, K_TB2_BARRIERS, K_WIDE, K_POST_SPLIT, K_COUNT };
+enum KnobId { K_TWO_STEP, K_TB2_PLANES, K_TB2_BARRIERS, K_WIDE, K_POST_SPLIT, K_MULTI, K_MULTI_DEPTH,
+              K_MULTI_TILE1, K_MULTI_TILE2, K_COUNT };
 struct KnobInit {
   KnobInit() {
     for (Knob& k : g_knobs) {
@@ -266,6 +278,121 @@ static int64_t two_step_pairs(bool two_step, int64_t nsteps) {
   return pairs;
 }
 
+// How the several-step kernel for 2D grids would run a pull run: the kernel,
+// its tile and the most steps per launch; fn == nullptr where it does not
+// apply.
+struct Tile2dChoice {
+  Tile2dFn fn = nullptr;
+  int t1 = 0, t2 = 0, steps = 0, reach = 1;
+};
+
+// Time of one launch in us, from the waves each CU issues: w[s] wavefronts per
+// tile in step s.  Fitted to 2600 timed launches on MI355X (13 grids of 64^2
+// to 2048^2 cells, 2 to 10 steps, tiles of 4 x 8 to 48 x 96; within 8-14 %
+// each, and the choice it makes within 5 % of the best one timed, 9 % at
+// 2048^2 FP16).  base: an empty launch; sync: one step's latency (loads or LDS,
+// arithmetic, barrier), once per round of resident blocks; issue: one
+// wavefront's step; load: one wavefront's loads of the input.
+struct Tile2dCost {
+  double base, sync, issue, load;
+};
+static double tile2d_cost(const Tile2dCost& c, int n1, int n2, int t1, int t2, int steps, int reach,
+                          int lds, int max_threads, int cu_lds, int cus) {
+  const int tiles = ((n1 + t1 - 1) / t1) * ((n2 + t2 - 1) / t2);
+  int waves = 0, first = 0;
+  for (int s = 0; s < steps; ++s) waves += first = ((t1 + 2 * reach * s) * (t2 + 2 * reach * s) + 63) / 64;
+  const int per_block = std::min(max_threads / 64, first);
+  const int resident = std::max(1, std::min(16, std::min(cu_lds / lds, 2 * (max_threads / 64) / per_block)));
+  const int per_cu = (tiles + cus - 1) / cus;
+  const int rounds = (per_cu + resident - 1) / resident;
+  return c.base + c.sync * (rounds * steps) + c.issue * ((double)waves * per_cu) +
+         c.load * ((double)first * per_cu);
+}
+
+// nsteps: the stages to run (see run_tiles)
+static Tile2dChoice tile2d_choice(const lbm_step_args* a, int64_t nsteps) {
+  Tile2dChoice ch;
+  const int mode = knob(K_MULTI);
+  if (mode == 0 || knob(K_TWO_STEP) == 0 || nsteps <= 2) return ch;
+  if (a->stencil != LBM_D2Q9 || a->streaming != LBM_PRE_STREAMING || a->n[0] != 1) return ch;
+  if (a->collision == LBM_COLL_LEARNED || a->n[1] * a->n[2] > 0x7fffffff) return ch;
+  if (a->stride[3] != 1 || (a->cell_class && a->stride[2] != a->n[2])) return ch;
+  const int bytes = storage_bytes(a->storage);
+  const int64_t last = a->stride[0] * 8 + a->stride[2] * (a->n[1] - 1) + a->n[2] - 1;
+  if (bytes <= 4 ? (last + 1) * bytes >= ((int64_t)1 << 32) : last >= 0x7fffffff) return ch;
+  int dev = 0, max_lds = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+    return ch;
+  const bool mask = a->cell_class != nullptr, kbc = a->collision == LBM_COLL_KBC;
+  if (mode != 2) {
+    // The row-sweeping two-step kernel computes each cell 1 + 4 / cx times,
+    // a tile more often; with boundaries (twice the overlap) or KBC (twice
+    // the arithmetic) it wins where it applies and its chunks of 8 rows fill
+    // the chip.  Measured in us per step, rows / tiles: 2048 x 512 channel
+    // KBC FP32 13.6 / 16.2, BGK 12.1 / 13.7, KBC FP16 14.1 / 14.9, periodic
+    // KBC 10.8 / 12.4, but BGK 9.3 / 9.2; 1536 x 512 channel KBC 13.9 / 13.1;
+    // 2048 x 256 10.6 / 9.0; 1024 x 1024 BGK FP16 19.5 / 12.1.  Knobs that ask
+    // for the two-step kernel get it.
+    int64_t lds = 0;
+    int nr = 0;
+    const bool rows = two_step_2d(a, &lds, &nr) != nullptr;
+    if (rows && (knob(K_TWO_STEP) == 2 || knob(K_TB2_PLANES) > 0)) return ch;
+    if (rows && (mask || kbc) && a->n[1] >= 8 * (int64_t)cus && a->n[2] >= 512) return ch;
+  }
+  ch.reach = mask ? 2 : 1;
+  static const int kTiles[][2] = {{8, 8},   {8, 16},  {12, 16}, {16, 16}, {8, 32},  {16, 32},
+                                  {24, 32}, {32, 32}, {16, 64}, {24, 48}, {32, 64}, {32, 96}};
+  static const int kSteps[] = {2, 3, 4, 5, 6, 8, 10};
+  const Tile2dCost cost = {mask ? 4.0 : (bytes == 8 ? 4.2 : 2.7),
+                           mask ? (kbc ? 0.64 : 1.1) : (bytes == 8 ? 0.58 : 0.74),
+                           kbc ? 0.085 : (bytes == 8 ? 0.048 : 0.024), 0.15};
+  const int64_t fixed = mask ? tile2d_static_lds_bytes() : 0;
+  double best = 0;
+  for (const int steps : kSteps) {
+    const int k = knob(K_MULTI_DEPTH) > 0 ? (int)std::min<int64_t>(knob(K_MULTI_DEPTH), nsteps) : steps;
+    if (k > nsteps) break;
+    for (const auto& t : kTiles) {
+      const int t1 = knob(K_MULTI_TILE1) > 0 ? knob(K_MULTI_TILE1) : t[0];
+      const int t2 = knob(K_MULTI_TILE2) > 0 ? knob(K_MULTI_TILE2) : t[1];
+      // one periodic wrap reaches every halo cell
+      const int m = ch.reach * (k - 1);
+      if (t1 + m > a->n[1] || t2 + m > a->n[2]) continue;
+      const int64_t lds = tile2d_lds_bytes(t1, t2, k, ch.reach, bytes, mask) + fixed;
+      if (lds > max_lds) continue;
+      const double us = tile2d_cost(cost, (int)a->n[1], (int)a->n[2], t1, t2, k, ch.reach, (int)lds,
+                                    bytes == 8 ? 512 : 1024, max_lds, cus) / k;
+      if (ch.steps == 0 || us < best) {
+        best = us;
+        ch.t1 = t1;
+        ch.t2 = t2;
+        ch.steps = k;
+      }
+    }
+  }
+  if (ch.steps == 0) return ch;
+  ch.fn = pick_tile2d_kernel(codec_id(a->storage, a->sr_seed), a->collision, mask);
+  return ch;
+}
+
+// Launches of a run of nsteps steps in `stages` stages, at most `most` each: as
+// few as keep the parity of nsteps, so that the result sits where single
+// steps leave it
+static int64_t tile2d_launches(int64_t nsteps, int64_t stages, int most) {
+  const int64_t n = (stages + most - 1) / most;
+  return n + ((nsteps - n) & 1);
+}
+
+// the same for a post-streaming run, which the kernel takes whole; stochastic
+// rounding is keyed to the launches of the split run (see lbm_run)
+static Tile2dChoice tile2d_post_choice(const lbm_step_args* a, int64_t nsteps) {
+  if (a->sr_seed != 0) return Tile2dChoice();
+  lbm_step_args k = *a;
+  k.streaming = LBM_PRE_STREAMING;
+  return tile2d_choice(&k, nsteps + 1);
+}
+
 // Validates the arguments and prepares the single-step kernel (one cell per
 // thread, block_tile indexing) of a step with a->streaming.
 static int prepare_step(const lbm_step_args* a, KParams& p, KernelFn& fn, dim3& grid, dim3& block) {
@@ -377,13 +504,55 @@ static void launch_singles(KernelFn fn, dim3 grid, dim3 block, KParams p, const 
   }
 }
 
+// A run of nsteps steps on the several-step kernel, from bufs[launch & 1]: pull
+// steps, or (post) steps in lettuce's default order, which are nsteps + 1
+// stages (see lbm_tile2d.hip).  The stages are spread evenly over the
+// launches.
+static void run_tiles(const lbm_step_args* a, const KParams& p, const Tile2dChoice& ch,
+                      const void* const (&bufs)[2], int64_t& launch, int64_t nsteps, bool post,
+                      uint32_t& step, hipStream_t s) {
+  const bool mask = a->cell_class != nullptr;
+  const int bytes = storage_bytes(a->storage);
+  Tile2dParams tp;
+  tp.k = p;
+  tp.t1 = ch.t1;
+  tp.t2 = ch.t2;
+  tp.reach = ch.reach;
+  tp.nt2 = (int)((a->n[2] + ch.t2 - 1) / ch.t2);
+  const unsigned nb = (unsigned)(tp.nt2 * ((a->n[1] + ch.t1 - 1) / ch.t1));
+  (void)hipFuncSetAttribute((const void*)ch.fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)tile2d_lds_bytes(ch.t1, ch.t2, ch.steps, ch.reach, bytes, mask));
+  const int64_t stages = post ? nsteps + 1 : nsteps;
+  const int64_t count = tile2d_launches(nsteps, stages, ch.steps);
+  for (int64_t k = 0; k < count; ++k, ++launch) {
+    tp.steps = (int)(stages / count + (k < stages % count ? 1 : 0));
+    tp.lead = post && k == 0;
+    tp.trail = post && k == count - 1;
+    const int m = ch.reach * (tp.steps - 1);
+    const int cells = (ch.t1 + 2 * m) * (ch.t2 + 2 * m);
+    const int threads = std::min(bytes == 8 ? 512 : 1024, (cells + 63) / 64 * 64);
+    tp.k.fin = bufs[launch & 1];
+    tp.k.fout = (void*)bufs[(launch + 1) & 1];
+    tp.k.sr_step = step;
+    step += (uint32_t)tp.steps;
+    hipLaunchKernelGGL(ch.fn, dim3(nb), dim3(threads),
+                       (size_t)tile2d_lds_bytes(ch.t1, ch.t2, tp.steps, ch.reach, bytes, mask), s, tp);
+  }
+}
+
 // `nsteps` pull steps of a (a->streaming == LBM_PRE_STREAMING) from
 // bufs[launch & 1]: pairs fused by the two-step kernel where it applies,
 // the rest as single steps.  The number of launches has the parity of
-// nsteps, so the result sits where single steps would leave it.
+// nsteps, so the result sits where single steps would leave it.  2D grids run
+// several steps per launch where tile2d_choice says so.
 static void run_pull_steps(const lbm_step_args* a, const KParams& p, KernelFn fn, dim3 grid,
                            dim3 block, const void* const (&bufs)[2], int64_t& launch,
                            int64_t nsteps, uint32_t& step, hipStream_t s) {
+  const Tile2dChoice ch = tile2d_choice(a, nsteps);
+  if (ch.fn) {
+    run_tiles(a, p, ch, bufs, launch, nsteps, false, step, s);
+    return;
+  }
   TbFn tb = two_step_kernel(a);
   int64_t lds = 0;
   int nr = 1;
@@ -534,6 +703,29 @@ int lbm_run_plan(const lbm_step_args* a, int64_t nsteps, int64_t* plan) {
   return LBM_OK;
 }
 
+int lbm_run_launches(const lbm_step_args* a, int64_t nsteps, int64_t* launches) {
+  if (!launches) return fail(LBM_E_ARG, "NULL launches");
+  int64_t plan[2];
+  int rc = lbm_run_plan(a, nsteps, plan);
+  if (rc) return rc;
+  launches[0] = 0;
+  launches[1] = plan[0];
+  launches[2] = plan[1];
+  const bool split = post_split(a, nsteps);
+  lbm_step_args k = *a;
+  k.streaming = LBM_PRE_STREAMING;
+  const bool whole = split && tile2d_post_choice(a, nsteps).fn;
+  const int64_t pull = split && !whole ? nsteps - 2 : nsteps, stages = whole ? nsteps + 1 : pull;
+  const Tile2dChoice ch =
+      split || a->streaming == LBM_PRE_STREAMING ? tile2d_choice(&k, stages) : Tile2dChoice();
+  if (ch.fn) {
+    launches[0] = tile2d_launches(pull, stages, ch.steps);
+    launches[1] = 0;
+    launches[2] = split && !whole ? 2 : 0;
+  }
+  return LBM_OK;
+}
+
 int lbm_run(const lbm_step_args* a, int64_t nsteps, void* stream) {
   if (nsteps < 0) return fail(LBM_E_ARG, "negative step count");
   KParams p;
@@ -558,6 +750,11 @@ int lbm_run(const lbm_step_args* a, int64_t nsteps, void* stream) {
     // (S C)^n = (S C S) (C S)^(n-2) C: collide only, n - 2 pull steps (two
     // fused per launch where the two-step kernel applies), then stream,
     // collide and stream.  n launches as with the push kernel, or fewer.
+    const Tile2dChoice ch = tile2d_post_choice(a, nsteps);
+    if (ch.fn) {
+      run_tiles(a, p, ch, bufs, launch, nsteps, true, step, s);
+      return check_launch("lbm_run (post-streaming)");
+    }
     lbm_step_args c = *a, k = *a, d = *a;
     c.streaming = LBM_NO_STREAMING;
     k.streaming = LBM_PRE_STREAMING;

@@ -397,13 +397,14 @@ __device__ __forceinline__ void outlet_neighbour(const KParams& p, const lbm_cel
 
 // The operator of a non-collision cell (one of LBM_OP_BOUNCE_BACK,
 // LBM_OP_EQUILIBRIUM, LBM_OP_OUTLET, LBM_OP_ANTI_BOUNCE_BACK, LBM_OP_KEEP)
-// on its populations f.  neighbour(K, g) fills g with the populations of
-// the neighbour x - K.dir as the streaming step leaves them (OUTLET,
-// ANTI_BOUNCE_BACK).
-template <class S, class ST, class NB>
+// on its populations f.  entry() is the cell's entry of the class table (in
+// LDS where the kernel staged it: from global memory it is two dependent
+// loads); neighbour(K, g) fills g with the populations of the neighbour
+// x - K.dir as the streaming step leaves them (OUTLET, ANTI_BOUNCE_BACK).
+template <class S, class ST, class CE, class NB>
 __device__ __forceinline__ void apply_boundary_op_nb(const KParams& p, uint32_t op, uint32_t flags,
                                                      int cell, typename ST::C (&f)[S::Q],
-                                                     NB&& neighbour) {
+                                                     CE&& entry, NB&& neighbour) {
   using C = typename ST::C;
   if (op == LBM_OP_BOUNCE_BACK) {
     // fullway bounce-back: f_q <- f_opp(q) (bounce_back_boundary.py:17-18)
@@ -414,7 +415,7 @@ __device__ __forceinline__ void apply_boundary_op_nb(const KParams& p, uint32_t 
     for (int q = 0; q < S::Q; ++q) f[q] = g[q];
   } else if (op == LBM_OP_EQUILIBRIUM) {
     // f <- feq(rho_bc, u_bc) (equilibrium_boundary_pu.py:79-84)
-    const lbm_cell_class& K = p.ct[p.cls[cell]];
+    const lbm_cell_class& K = entry();
     C rho, u[3];
     if (flags & LBM_CLASS_BC_FIELD) {
       rho = (C)p.bcf[cell];
@@ -430,7 +431,7 @@ __device__ __forceinline__ void apply_boundary_op_nb(const KParams& p, uint32_t 
     equilibrium<S, C>(rho, u, f);
   } else if (op == LBM_OP_OUTLET) {
     // f <- feq(rho_out, u(x - dir)) (equilibrium_outlet_p.py:63-73)
-    const lbm_cell_class& K = p.ct[p.cls[cell]];
+    const lbm_cell_class& K = entry();
     C g[S::Q];
     neighbour(K, g);
     C rho_n, u[3];
@@ -441,7 +442,7 @@ __device__ __forceinline__ void apply_boundary_op_nb(const KParams& p, uint32_t 
     // populations v leaving through the outlet (e_v . dir = 1),
     // f_opp(v) <- -f_v + w_v rho (2 + (e_v.u_w)^2 / cs^4 - |u_w|^2 / cs^2)
     // with u_w = u + (u - u(x - dir)) / 2 and rho, u of the cell itself
-    const lbm_cell_class& K = p.ct[p.cls[cell]];
+    const lbm_cell_class& K = entry();
     C g[S::Q];
     neighbour(K, g);
     C rho, u[3], rho_n, un[3];
@@ -468,6 +469,7 @@ __device__ __forceinline__ void apply_boundary_op(const KParams& p, uint32_t op,
                                                   int cell, int i0, int i1, int i2,
                                                   typename ST::C (&f)[S::Q]) {
   apply_boundary_op_nb<S, ST>(p, op, flags, cell, f,
+                              [&]() -> const lbm_cell_class& { return p.ct[p.cls[cell]]; },
                               [&](const lbm_cell_class& K, typename ST::C(&g)[S::Q]) {
                                 outlet_neighbour<S, ST, PULL>(p, K, i0, i1, i2, g);
                               });
