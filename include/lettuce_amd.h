@@ -379,6 +379,20 @@ int lbm_learned_train_backward(int32_t stencil, int32_t storage, const int64_t n
                                int32_t lam_gathered, void* mu, void* record,
                                void* stream);
 
+/* lbm_learned_train_backward and the parameter gradient of the same step in
+ * one pass, for F32: mu as there, and grad [LBM_LEARNED_PARAMS] (F32, the
+ * parameter layout above) += the gradient, without a record.  workspace holds
+ * lbm_learned_gradient_workspace(storage, cells) bytes of per-block partial
+ * sums, added in a fixed order (deterministic); -1 for an unsupported storage
+ * or cells < 1. */
+int64_t lbm_learned_gradient_workspace(int32_t storage, int64_t cells);
+int lbm_learned_train_gradient(int32_t stencil, int32_t storage, const int64_t n[3],
+                               double tau, const void* params, double in_scale,
+                               double rate_lo, double rate_hi,
+                               const void* f_in, const void* lam,
+                               int32_t lam_gathered, void* mu, void* workspace,
+                               void* grad, void* stream);
+
 /* lam_q(x) = mu_q(x + e_q): the adjoint of periodic pull streaming (the
  * gradient with respect to the populations before the step) */
 int lbm_unpull(int32_t stencil, int32_t storage, const int64_t n[3], const void* mu,

@@ -105,6 +105,9 @@ _SIGNATURES = {
                                    _vp], ctypes.c_int),
     "lbm_learned_train_backward": ([_i32, _i32, _vp, _dbl, _vp, _dbl, _dbl, _dbl, _vp, _vp,
                                     _i32, _vp, _vp, _vp], ctypes.c_int),
+    "lbm_learned_gradient_workspace": ([_i32, _i64], _i64),
+    "lbm_learned_train_gradient": ([_i32, _i32, _vp, _dbl, _vp, _dbl, _dbl, _dbl, _vp, _vp,
+                                    _i32, _vp, _vp, _vp, _vp], ctypes.c_int),
     "lbm_unpull": ([_i32, _i32, _vp, _vp, _vp, _vp], ctypes.c_int),
     "lbm_learned_grad_workspace": ([_i32, _i64], _i64),
     "lbm_learned_grad_reduce": ([_i32, _i64, _vp, _vp, _vp, _vp], ctypes.c_int),

@@ -13,8 +13,9 @@ does not record a graph; it runs the adjoint kernels of csrc/lbm_train.hip:
   mu_n          = (dC/dg)^T lambda_{n+1}     per cell (lbm_learned_train_backward)
   lambda_n,q(x) = mu_n,q(x + e_q)            transpose of the pull, fused into
                                              the next backward launch
-  dL/dtheta    += sum over cells of outer products of the per-cell record,
-                  one GEMM per step
+  dL/dtheta    += sum over cells of outer products of the MLP's activations
+                  and their adjoints (FP32: in the adjoint's kernel,
+                  lbm_learned_train_gradient; FP64: from a per-cell record)
 
 States are kept every `checkpoint_every` steps and the steps between two
 kept states are recomputed during the backward pass, so the memory is
@@ -125,11 +126,26 @@ class _Problem:
             record.data_ptr() if record is not None else None, self.stream),
             "lbm_learned_train_backward")
 
+    @property
+    def fused_gradient(self):
+        """FP32: the adjoint and the parameter gradient run as one kernel"""
+        return self.storage == N.F32
+
+    def adjoint_gradient(self, f, lam, gathered, mu, workspace, grad):
+        """mu of adjoint(), and grad [LEARNED_PARAMS] += the parameter gradient"""
+        c = self.cfg
+        N.check(N.lib().lbm_learned_train_gradient(
+            self.stencil, self.storage, self.n, c.tau, self.theta.data_ptr(), c.in_scale, c.rate_lo,
+            c.rate_hi, f.data_ptr(), lam.data_ptr(), int(gathered), mu.data_ptr(),
+            workspace.data_ptr(), grad.data_ptr(), self.stream), "lbm_learned_train_gradient")
+
     def grad_workspace(self):
-        """the per-block partial sums of lbm_learned_grad_reduce"""
-        nbytes = N.lib().lbm_learned_grad_workspace(self.storage, self.cells)
+        """the per-block partial sums of the parameter gradient"""
+        fn = (N.lib().lbm_learned_gradient_workspace if self.fused_gradient
+              else N.lib().lbm_learned_grad_workspace)
+        nbytes = fn(self.storage, self.cells)
         if nbytes < 0:
-            raise RuntimeError("lbm_learned_grad_workspace rejected the arguments")
+            raise RuntimeError("the gradient workspace rejected the arguments")
         return torch.empty(nbytes // self.theta.element_size(), dtype=self.theta.dtype,
                            device=self.theta.device)
 
@@ -169,10 +185,11 @@ class LearnedRollout(torch.autograd.Function):
         lam = grad_out.to(prob.theta.dtype).contiguous()
         gathered = False
         mu = [torch.empty_like(lam), torch.empty_like(lam)]
-        record = torch.empty((N.LEARNED_RECORD, prob.cells), dtype=lam.dtype, device=lam.device)
         need_theta = ctx.needs_input_grad[1]
-        # the parameter gradient, summed over the cells of every step's
-        # record by lbm_learned_grad_reduce
+        record = torch.empty((N.LEARNED_RECORD, prob.cells), dtype=lam.dtype, device=lam.device) \
+            if need_theta and not prob.fused_gradient else None
+        # the parameter gradient, summed over the cells of every step: in the
+        # adjoint's own kernel (FP32) or from its record (FP64)
         grad_theta = torch.zeros(N.LEARNED_PARAMS, dtype=lam.dtype, device=lam.device) \
             if need_theta else None
         workspace = prob.grad_workspace() if need_theta else None
@@ -187,9 +204,12 @@ class LearnedRollout(torch.autograd.Function):
                 states.append(nxt)
             for i in reversed(range(length)):
                 out = mu[k & 1]
-                prob.adjoint(states[i], lam, gathered, out, record if need_theta else None)
-                if need_theta:
-                    prob.grad_reduce(record, workspace, grad_theta)
+                if need_theta and prob.fused_gradient:
+                    prob.adjoint_gradient(states[i], lam, gathered, out, workspace, grad_theta)
+                else:
+                    prob.adjoint(states[i], lam, gathered, out, record)
+                    if need_theta:
+                        prob.grad_reduce(record, workspace, grad_theta)
                 lam, gathered, k = out, True, k + 1
             states.clear()
         grad_f0 = None
