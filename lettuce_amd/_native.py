@@ -164,7 +164,7 @@ def check(rc, what):
 class tuning:
     """Context manager that sets launch-tuning knobs of the library
     (lbm_set_tuning: two_step, two_step_planes, two_step_barriers,
-    wide_offsets, post_split, multi_step, multi_step_depth, multi_step_tile1,
+    wide_offsets, post_split, flat, multi_step, multi_step_depth, multi_step_tile1,
     multi_step_tile2) and restores their start values on exit.
     The knobs are process-wide; they exist for measurements and tests."""
 

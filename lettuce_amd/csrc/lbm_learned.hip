@@ -505,7 +505,7 @@ __global__ void __launch_bounds__(256, 3) learned_kernel(const KParams p, const 
       }
     } else {
       if constexpr (RAW) shift_all(f, C(1));
-      apply_boundary_op<S, ST, PULL>(p, op, flags, cell, i0, i1, i2, f);
+      apply_boundary_op<S, ST, PULL>(p, ctl, op, flags, cell, i0, i1, i2, f);
       if constexpr (RAW) shift_all(f, C(-1));
     }
     if (out_of_grid) continue;

@@ -1,6 +1,9 @@
 // The fused stream + collide kernel.  One thread owns one cell; a block is a
 // run of cells along the contiguous axis i2, so every population load and
-// store of a wavefront is one coalesced 256-byte (FP32) transaction.
+// store of a wavefront is one coalesced 256-byte (FP32) transaction.  Where
+// the rows are no whole number of wavefronts and follow each other in memory
+// (FLAT), a block is a run of cells across rows instead: no lane idles and the
+// stores fill whole cache lines.
 //
 // Streaming follows lettuce's semantics exactly:
 //  - pre-streaming (pull), lettuce/_simulation.py:241-256:
@@ -38,7 +41,21 @@ struct KParams {
   int nclasses = 0;       // entries of ct (0 without boundaries)
   uint32_t sr_seed = 0;   // stochastic rounding of BF16 storage (0: to nearest)
   uint32_t sr_step = 0;   // step index of the launch (its first step)
+  uint32_t div2 = 0, div1 = 0;  // FLAT: n2 and n1 as divisors (see fast_div)
+  int shift2 = 0, shift1 = 0;
 };
+
+// c / n for c < 2^31 by a multiplication with n's reciprocal, rounded up:
+// m = ceil(2^(31 + s) / n) with 2^(s - 1) < n <= 2^s leaves
+// c (m n - 2^(31 + s)) < 2^31 n <= 2^(31 + s), so the floor is exact; m < 2^32
+inline void set_divisor(uint32_t n, uint32_t& m, int& s) {
+  s = 0;
+  while ((1u << s) < n) ++s;
+  m = (uint32_t)((((uint64_t)1 << (31 + s)) + n - 1) / n);
+}
+__host__ __device__ inline uint32_t fast_div(uint32_t c, uint32_t m, int s) {
+  return (uint32_t)(((uint64_t)c * m) >> 31) >> s;
+}
 
 // One stored element: to nearest, or with stochastic rounding when the
 // format supports it and the run asks for it (key: sr_step_key of the
@@ -136,40 +153,52 @@ __device__ __forceinline__ typename ST::C shift_of(double w, const KParams& p) {
   return ST::shifted ? (C)(w * p.rho0) : C(0);
 }
 
-__device__ __forceinline__ bool cls_solid(const KParams& p, int cell) {
-  return (p.ct[p.cls[cell]].flags & LBM_CLASS_SOLID) != 0;
-}
-
-// Post-streaming populations of the cell at offset `cell` whose neighbour
-// tables are a0/a1/a2, with the cell's own class fields (nsm, flags).
-template <class S, class ST, bool MASK>
-__device__ __forceinline__ void gather_pull(const KParams& p, int cell,
-                                            const long long (&a0)[3], const int (&a1)[3],
-                                            const int (&a2)[3], uint32_t nsm,
-                                            uint32_t flags, typename ST::C (&f)[S::Q]) {
+// The pull of a cell on a grid without boundaries, whose neighbour tables are
+// a0/a1/a2.
+template <class S, class ST, class X>
+__device__ __forceinline__ void gather_pull(const KParams& p, const X (&a0)[3], const int (&a1)[3],
+                                            const int (&a2)[3], typename ST::C (&f)[S::Q]) {
   using T = typename ST::T;
   const T* fin = (const T*)p.fin;
 #pragma unroll
   for (int q = 0; q < S::Q; ++q) {
-    const typename ST::C sh = shift_of<ST>(S::w[q], p);
-    if (!MASK) {
-      const long long plane = nb_plane<S>(q, -1, a0);
-      f[q] = ST::ld(at_plane(fin + q * p.sq, plane), in_plane(plane, nb_in_plane<S>(q, -1, a1, a2)),
-                    sh);
-    } else {
-      const int src = nb_offset<S>(q, -1, a0, a1, a2);
-      bool hw = false;
-      if ((flags & (LBM_CLASS_NEAR_SOLID | LBM_CLASS_SOLID)) == LBM_CLASS_NEAR_SOLID && q != 0)
-        hw = cls_solid(p, src);
-      if (hw) {
-        const int o = S::opp[q];
-        f[q] = ST::ld(fin + o * p.sq, cell, shift_of<ST>(S::w[o], p));
-      } else {
-        const int idx = ((nsm >> q) & 1u) ? cell : src;
-        f[q] = ST::ld(fin + q * p.sq, idx, sh);
-      }
-    }
+    const X plane = nb_plane<S>(q, -1, a0);
+    f[q] = ST::ld(at_plane(fin + q * p.sq, plane), in_plane(plane, nb_in_plane<S>(q, -1, a1, a2)),
+                  shift_of<ST>(S::w[q], p));
   }
+}
+
+// The same with the rules of the cell's class, for single cells: the class ids
+// of the sources in one round of loads, then the populations they select.  ct:
+// the class table (in LDS or global memory).
+template <class S, class ST>
+__device__ __forceinline__ void gather_pull_masked(const KParams& p, const lbm_cell_class* ct,
+                                                   int cell, const long long (&a0)[3],
+                                                   const int (&a1)[3], const int (&a2)[3],
+                                                   typename ST::C (&f)[S::Q]) {
+  using T = typename ST::T;
+  const T* fin = (const T*)p.fin;
+  uint32_t cid[S::Q];
+#pragma unroll
+  for (int q = 0; q < S::Q; ++q) cid[q] = p.cls[nb_offset<S>(q, -1, a0, a1, a2)];
+  __builtin_amdgcn_sched_barrier(0);
+  const lbm_cell_class& K = ct[cid[0]];  // e_0 = 0: the cell itself
+  const uint32_t nsm = K.no_stream;
+  const bool near = (K.flags & (LBM_CLASS_NEAR_SOLID | LBM_CLASS_SOLID)) == LBM_CLASS_NEAR_SOLID;
+  uint32_t solid = 0;
+#pragma unroll
+  for (int q = 1; q < S::Q; ++q) solid |= (ct[cid[q]].flags & LBM_CLASS_SOLID) ? 1u << q : 0u;
+  if (!near) solid = 0;
+  T raw[S::Q];
+#pragma unroll
+  for (int q = 0; q < S::Q; ++q) {
+    const bool bounce = (solid >> q) & 1u;
+    const int idx = bounce || ((nsm >> q) & 1u) ? cell : nb_offset<S>(q, -1, a0, a1, a2);
+    raw[q] = fin[(bounce ? S::opp[q] : q) * p.sq + idx];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int q = 0; q < S::Q; ++q) f[q] = ST::dec(raw[q], shift_of<ST>(S::w[q], p));
 }
 
 // The first p.nclasses entries of the cell-class table, copied into LDS by
@@ -372,10 +401,13 @@ __device__ __forceinline__ void collide(C (&f)[S::Q], const CollParams<C>& cp) {
 
 // Populations of the neighbour x - dir of an outlet cell as the streaming
 // step leaves them (its moments are those of its post-collision state when
-// it collides with a momentum-conserving operator).
+// it collides with a momentum-conserving operator).  The outlet is the last
+// plane of a grid that flows along i0: what its cells wait for adds to the
+// launch (18 populations one class lookup after the other: 12 us of 63 at
+// 192 x 96 x 96, D3Q19 FP32).
 template <class S, class ST, bool PULL>
-__device__ __forceinline__ void outlet_neighbour(const KParams& p, const lbm_cell_class& K,
-                                                 int i0, int i1, int i2,
+__device__ __forceinline__ void outlet_neighbour(const KParams& p, const lbm_cell_class* ct,
+                                                 const lbm_cell_class& K, int i0, int i1, int i2,
                                                  typename ST::C (&g)[S::Q]) {
   const int j0 = i0 - K.dir[0], j1 = i1 - K.dir[1], j2 = i2 - K.dir[2];
   const int w0 = j0 < 0 ? j0 + p.n0 : (j0 >= p.n0 ? j0 - p.n0 : j0);
@@ -388,8 +420,7 @@ __device__ __forceinline__ void outlet_neighbour(const KParams& p, const lbm_cel
   axis_offsets(w2, p.n2, 1, c2);
   const int nb = (int)(c0[1] + c1[1] + c2[1]);
   if (PULL) {
-    const lbm_cell_class& KN = p.ct[p.cls[nb]];
-    gather_pull<S, ST, true>(p, nb, c0, c1, c2, KN.no_stream, KN.flags, g);
+    gather_pull_masked<S, ST>(p, ct, nb, c0, c1, c2, g);
   } else {
     gather_own<S, ST>(p, 0, nb, g);
   }
@@ -464,14 +495,15 @@ __device__ __forceinline__ void apply_boundary_op_nb(const KParams& p, uint32_t 
   // LBM_OP_KEEP: unchanged
 }
 
+// ct: the class table (in LDS or global memory)
 template <class S, class ST, bool PULL>
-__device__ __forceinline__ void apply_boundary_op(const KParams& p, uint32_t op, uint32_t flags,
-                                                  int cell, int i0, int i1, int i2,
-                                                  typename ST::C (&f)[S::Q]) {
+__device__ __forceinline__ void apply_boundary_op(const KParams& p, const lbm_cell_class* ct,
+                                                  uint32_t op, uint32_t flags, int cell, int i0,
+                                                  int i1, int i2, typename ST::C (&f)[S::Q]) {
   apply_boundary_op_nb<S, ST>(p, op, flags, cell, f,
-                              [&]() -> const lbm_cell_class& { return p.ct[p.cls[cell]]; },
+                              [&]() -> const lbm_cell_class& { return ct[p.cls[cell]]; },
                               [&](const lbm_cell_class& K, typename ST::C(&g)[S::Q]) {
-                                outlet_neighbour<S, ST, PULL>(p, K, i0, i1, i2, g);
+                                outlet_neighbour<S, ST, PULL>(p, ct, K, i0, i1, i2, g);
                               });
 }
 
@@ -518,14 +550,15 @@ __device__ __forceinline__ void store_cell(const KParams& p, int cell, const X (
       // (b) the cell's own slot q
       bool own_bounce = false;
       if (q != 0 && !self_solid && (flags & LBM_CLASS_NEAR_SOLID))
-        own_bounce = cls_solid(p, nb_offset<S>(q, -1, a0, a1, a2));
+        own_bounce = (p.ct[p.cls[nb_offset<S>(q, -1, a0, a1, a2)]].flags & LBM_CLASS_SOLID) != 0;
       if (own_bounce) store_elem<ST>(p, fout + q * p.sq, cell, f[S::opp[q]], sh, key, cell, q);
       else if ((nsm >> q) & 1u) store_elem<ST>(p, fout + q * p.sq, cell, f[q], sh, key, cell, q);
     }
   }
 }
 
-template <class S, class ST, int COLL, bool MASK, int MODE>
+// FLAT: each population's rows are contiguous and its byte offsets fit 32 bits
+template <class S, class ST, int COLL, bool MASK, int MODE, bool FLAT>
 __global__ void __launch_bounds__(256) step_kernel(const KParams p) {
   using C = typename ST::C;
   using T = typename ST::T;
@@ -539,14 +572,25 @@ __global__ void __launch_bounds__(256) step_kernel(const KParams p) {
     __syncthreads();
   }
 
-  int i0, i1, b2;
-  block_tile(p, blockIdx.x, i0, i1, b2);
-  const int i2 = b2 * blockDim.x + threadIdx.x;
-  if (i2 >= p.n2) return;
+  using X = std::conditional_t<FLAT, int, long long>;
+  int i0, i1, i2;
+  if constexpr (FLAT) {
+    const uint32_t c = blockIdx.x * 256u + threadIdx.x;
+    if (c >= (uint32_t)p.ncells) return;
+    const uint32_t r = fast_div(c, p.div2, p.shift2);
+    i2 = (int)(c - r * (uint32_t)p.n2);
+    i0 = (int)fast_div(r, p.div1, p.shift1);
+    i1 = (int)(r - (uint32_t)i0 * (uint32_t)p.n1);
+  } else {
+    int b2;
+    block_tile(p, blockIdx.x, i0, i1, b2);
+    i2 = b2 * blockDim.x + threadIdx.x;
+    if (i2 >= p.n2) return;
+  }
 
-  long long a0[3];
+  X a0[3];
   int a1[3], a2[3];
-  axis_offsets(i0, p.n0, p.s0, a0);
+  axis_offsets(i0, p.n0, (X)p.s0, a0);
   axis_offsets(i1, p.n1, p.s1, a1);
   axis_offsets(i2, p.n2, 1, a2);
   const int cell = (int)(a0[1] + a1[1] + a2[1]);  // used with boundaries only
@@ -556,14 +600,16 @@ __global__ void __launch_bounds__(256) step_kernel(const KParams p) {
   if (MASK) {
     gather_batched<S, ST, MASK, PULL>(p, cell, a0, a1, a2, ctl, nsm, flags, op, f);
   } else if (PULL) {
-    gather_pull<S, ST, MASK>(p, cell, a0, a1, a2, nsm, flags, f);
+    gather_pull<S, ST>(p, a0, a1, a2, f);
+  } else if (FLAT) {
+    gather_own<S, ST>(p, 0, cell, f);
   } else {
     gather_own<S, ST>(p, a0[1], a1[1] + a2[1], f);
   }
 
   const CollParams<C> cp = coll_params<C>(p);
   if (!MASK || op == LBM_OP_COLLIDE) collide<S, C, COLL>(f, cp);
-  else apply_boundary_op<S, ST, PULL>(p, op, flags, cell, i0, i1, i2, f);
+  else apply_boundary_op<S, ST, PULL>(p, ctl, op, flags, cell, i0, i1, i2, f);
   store_cell<S, ST, MASK, PUSH>(p, cell, a0, a1, a2, nsm, flags, f);
 }
 
@@ -595,44 +641,45 @@ __device__ __forceinline__ T wave_shift(T v) {
 // ---------------------------------------------------------------------------
 using KernelFn = void (*)(const KParams);
 
-template <class S, class ST, int COLL, bool MASK>
+template <class S, class ST, int COLL, bool MASK, bool FLAT>
 KernelFn pick_mode(int mode) {
   switch (mode) {
-    case 0: return step_kernel<S, ST, COLL, MASK, 0>;
-    case 1: return step_kernel<S, ST, COLL, MASK, 1>;
-    case 2: return step_kernel<S, ST, COLL, MASK, 2>;
-    case 3: return step_kernel<S, ST, COLL, MASK, 3>;
+    case 0: return step_kernel<S, ST, COLL, MASK, 0, FLAT>;
+    case 1: return step_kernel<S, ST, COLL, MASK, 1, FLAT>;
+    case 2: return step_kernel<S, ST, COLL, MASK, 2, FLAT>;
+    case 3: return step_kernel<S, ST, COLL, MASK, 3, FLAT>;
   }
   return nullptr;
 }
 
 template <class S, class ST, int COLL>
-KernelFn pick_mask(bool mask, int mode) {
-  return mask ? pick_mode<S, ST, COLL, true>(mode) : pick_mode<S, ST, COLL, false>(mode);
+KernelFn pick_mask(bool mask, int mode, bool flat) {
+  if (flat) return mask ? pick_mode<S, ST, COLL, true, true>(mode) : pick_mode<S, ST, COLL, false, true>(mode);
+  return mask ? pick_mode<S, ST, COLL, true, false>(mode) : pick_mode<S, ST, COLL, false, false>(mode);
 }
 
 template <class S, class ST>
-KernelFn pick_coll(int coll, bool mask, int mode) {
+KernelFn pick_coll(int coll, bool mask, int mode, bool flat) {
   switch (coll) {
-    case LBM_COLL_NONE: return pick_mask<S, ST, LBM_COLL_NONE>(mask, mode);
-    case LBM_COLL_BGK: return pick_mask<S, ST, LBM_COLL_BGK>(mask, mode);
-    case LBM_COLL_TRT: return pick_mask<S, ST, LBM_COLL_TRT>(mask, mode);
-    case LBM_COLL_BGK_GUO: return pick_mask<S, ST, LBM_COLL_BGK_GUO>(mask, mode);
+    case LBM_COLL_NONE: return pick_mask<S, ST, LBM_COLL_NONE>(mask, mode, flat);
+    case LBM_COLL_BGK: return pick_mask<S, ST, LBM_COLL_BGK>(mask, mode, flat);
+    case LBM_COLL_TRT: return pick_mask<S, ST, LBM_COLL_TRT>(mask, mode, flat);
+    case LBM_COLL_BGK_GUO: return pick_mask<S, ST, LBM_COLL_BGK_GUO>(mask, mode, flat);
     case LBM_COLL_KBC:
       if constexpr (S::ID == LBM_D3Q19) return nullptr;  // lettuce: D2Q9/D3Q27 only
-      else return pick_mask<S, ST, LBM_COLL_KBC>(mask, mode);
+      else return pick_mask<S, ST, LBM_COLL_KBC>(mask, mode, flat);
   }
   return nullptr;
 }
 
 template <class S>
-KernelFn pick_kernel(int storage, int coll, bool mask, int mode) {
+KernelFn pick_kernel(int storage, int coll, bool mask, int mode, bool flat) {
   switch (storage) {
-    case LBM_F32: return pick_coll<S, StF32>(coll, mask, mode);
-    case LBM_F64: return pick_coll<S, StF64>(coll, mask, mode);
-    case LBM_F16_SHIFTED: return pick_coll<S, StF16>(coll, mask, mode);
-    case LBM_BF16_SHIFTED: return pick_coll<S, StBF16>(coll, mask, mode);
-    case kCodecBF16SR: return pick_coll<S, StBF16SR>(coll, mask, mode);
+    case LBM_F32: return pick_coll<S, StF32>(coll, mask, mode, flat);
+    case LBM_F64: return pick_coll<S, StF64>(coll, mask, mode, flat);
+    case LBM_F16_SHIFTED: return pick_coll<S, StF16>(coll, mask, mode, flat);
+    case LBM_BF16_SHIFTED: return pick_coll<S, StBF16>(coll, mask, mode, flat);
+    case kCodecBF16SR: return pick_coll<S, StBF16SR>(coll, mask, mode, flat);
   }
   return nullptr;
 }

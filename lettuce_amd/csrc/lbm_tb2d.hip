@@ -174,7 +174,7 @@ __global__ void __launch_bounds__(1024) tb2d_kernel(const Tb2dParams P) {
       }
     }
     if (op == LBM_OP_COLLIDE) collide<S, C, COLL>(f, cp);
-    else apply_boundary_op<S, ST, true>(p, op, flags, cell, 0, wrap(x0 - H + rc, p.n1), y, f);
+    else apply_boundary_op<S, ST, true>(p, p.ct, op, flags, cell, 0, wrap(x0 - H + rc, p.n1), y, f);
     const int slot = rc % R;
     const uint32_t hs = sr ? sr_cell(key1, (uint32_t)cell) : 0u;
 #pragma unroll

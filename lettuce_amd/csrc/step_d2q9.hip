@@ -2,7 +2,7 @@
 #include "lbm_step_impl.h"
 
 namespace lbm {
-KernelFn pick_kernel_d2q9(int storage, int coll, bool mask, int mode) {
-  return pick_kernel<D2Q9>(storage, coll, mask, mode);
+KernelFn pick_kernel_d2q9(int storage, int coll, bool mask, int mode, bool flat) {
+  return pick_kernel<D2Q9>(storage, coll, mask, mode, flat);
 }
 }  // namespace lbm

@@ -1,0 +1,71 @@
+"""Single steps with blocks that run across rows (step_kernel's FLAT, for rows
+that are no multiple of 64 cells) against the same steps row by row: the cell
+arithmetic is the same code, so the states agree bit for bit without
+collision and to its rounding with one.  Extents of one cell, rows shorter
+and longer than a wavefront, a last block with few cells, every storage
+format, streaming order and stencil, with and without boundaries."""
+import numpy as np
+import pytest
+import torch
+
+import lettuce_amd as lt
+from tests.test_parity_gpu import ArrayFlow
+from tests.test_two_step_2d_gpu import COLLISIONS, ULPS
+
+pytestmark = pytest.mark.gpu
+
+F32, F64 = torch.float32, torch.float64
+PRE, POST = lt.StreamingStrategy.PRE_STREAMING, lt.StreamingStrategy.POST_STREAMING
+TOL = dict(ULPS, f64=4 * 0.5 * 2.0 ** -52)
+
+
+def _f0(stencil, res):
+    g = torch.Generator().manual_seed(sum(res))
+    w = torch.tensor(stencil.w, dtype=F64).reshape([-1] + [1] * len(res))
+    return w * (1 + 0.05 * torch.rand([stencil.q] + res, generator=g, dtype=F64))
+
+
+def _solid(res):
+    """a body near the inlet"""
+    grid = np.meshgrid(*[np.arange(n) for n in res], indexing="ij")
+    return sum((x - n / (3 if a == 0 else 2)) ** 2 for a, (x, n) in enumerate(zip(grid, res))) < 9
+
+
+@pytest.mark.parametrize("stencil,res,storage,coll,channel,order", [
+    ("D3Q19", [1, 1, 5], "f32", "none", False, PRE),
+    ("D3Q19", [5, 1, 65], "f32", "none", False, POST),
+    ("D3Q19", [21, 13, 30], "f32", "bgk", False, PRE),
+    ("D3Q27", [7, 9, 127], "f16_shifted", "kbc", False, POST),
+    ("D3Q27", [6, 17, 1], "bf16_shifted", "none", False, PRE),
+    ("D3Q19", [11, 8, 90], "f64", "trt", False, POST),
+    ("D2Q9", [33, 50], "f32", "kbc", False, POST),
+    ("D3Q19", [20, 13, 30], "f64", "none", True, POST),
+    ("D3Q19", [20, 13, 96], "f32", "bgk", True, PRE),
+    ("D3Q27", [19, 12, 31], "f32", "none", True, PRE),
+    ("D2Q9", [40, 21], "f16_shifted", "bgk", True, PRE)])
+def test_flat_matches_rows(stencil, res, storage, coll, channel, order, knobs):
+    S = getattr(lt, stencil)()
+    dtype = F64 if storage == "f64" else F32
+    f0 = _f0(S, res).numpy()
+    out = []
+    for flat in (0, 1):
+        knobs(two_step=0)
+        knobs(flat=flat)
+        ctx = lt.Context("cuda:0", dtype=dtype, storage=storage)
+        if channel:
+            flow = lt.Obstacle(ctx, res, 50, 0.1, domain_length_x=res[0] / 6, stencil=S,
+                               outlet="equilibrium", solid="halfway", walls=True)
+            flow.mask = _solid(res)
+            flow.f = torch.from_numpy(f0)
+        else:
+            flow = ArrayFlow(ctx, f0, S)
+        sim = lt.Simulation(flow, COLLISIONS[coll](0.7), [], order)
+        sim(5)
+        torch.cuda.synchronize()
+        out.append((flow._state.detach().cpu().contiguous().view(-1).view(torch.uint8).numpy(),
+                    flow.f.double().cpu().numpy()))
+    if coll == "none":
+        assert np.array_equal(out[0][0], out[1][0])
+    else:
+        tol = 5 * TOL[storage] * (50 if coll == "kbc" else 1)
+        assert np.abs(out[0][1] - out[1][1]).max() <= tol
