@@ -396,6 +396,17 @@ static Tile2dChoice tile2d_post_choice(const lbm_step_args* a, int64_t nsteps) {
   return tile2d_choice(&k, nsteps + 1);
 }
 
+// Whether both population arrays stay in the device's 256 MB last-level cache
+// from one launch to the next.  The stores then go through the caches; larger
+// arrays are streamed past them, since what a launch writes is gone before the
+// next one reads it.  Measured on MI355X, us per step, past / through: D3Q19
+// FP32 150 x 100 x 90 (205 MB) 40.2 / 34.1, 192 x 96 x 96 (269 MB) 50.5 / 43.9,
+// 128^3 (319 MB) 66.6 / 62.2, 130^3 (334 MB) 66.4 / 67.6, 200^3 (1.2 GB)
+// 214 / 225, D2Q9 2000^2 (288 MB) 51.9 / 49.6.
+static bool fits_cache(const lbm_step_args* a, int64_t limit) {
+  return 2 * a->n[0] * a->n[1] * a->n[2] * stencil_q(a->stencil) * storage_bytes(a->storage) <= limit;
+}
+
 // Whether single steps take blocks across rows (step_kernel's FLAT): rows that
 // are no whole number of wavefronts, stored one after the other, with byte
 // offsets within 32 bits.  Blocks of one row leave lanes idle there (90 cells
@@ -509,6 +520,7 @@ static int prepare_step(const lbm_step_args* a, KParams& p, KernelFn& fn, dim3& 
   p.rho0 = (a->storage == LBM_F16_SHIFTED || a->storage == LBM_BF16_SHIFTED) ? a->rho0_shift : 0.0;
   p.sr_seed = a->sr_seed;
   p.sr_step = a->sr_step;
+  p.cached = fits_cache(a, 300000000);
   grid = dim3((unsigned)nb);
   block = dim3(bs);
   return LBM_OK;
@@ -538,6 +550,8 @@ static void run_tiles(const lbm_step_args* a, const KParams& p, const Tile2dChoi
   const int bytes = storage_bytes(a->storage);
   Tile2dParams tp;
   tp.k = p;
+  // (FP64 1024^2, 151 MB: 17.6 / 17.3, FP32 2000^2, 288 MB: 29.9 / 31.9)
+  tp.k.cached = fits_cache(a, 200000000);
   tp.t1 = ch.t1;
   tp.t2 = ch.t2;
   tp.reach = ch.reach;
@@ -615,34 +629,38 @@ static void run_pull_steps(const lbm_step_args* a, const KParams& p, KernelFn fn
     tp.k = p;
     tp.nzt = (int)(a->n[2] / 64);
     tp.nyt = (int)(a->n[1] / TB_Y);
-    // x chunk: 64 planes, or 128 where 64-plane tiles would make between one
-    // and two rounds of the blocks the device holds at once, so that they
-    // make one (or 48, below).  Measured on MI355X: D3Q19 256^3 (512 tiles, 512 resident
-    // blocks) and 1024^3 (32768 tiles) are fastest at 64 planes (larger
-    // chunks: -4 % to -17 %); D3Q27 KBC FP32 256^3, one block per CU, runs
-    // 30.7k MLUPS at 64 planes and 31.3k at 128.
+    // x chunk: a block sweeps cx + 2 planes, and a CU's share of the blocks
+    // takes as long as its planes, a few per cent more where it has only one
+    // block to hide latency with although two fit.  The chunk that gives the
+    // fullest CU the fewest planes, then.  Measured on MI355X in us per step,
+    // 64 planes / chosen: D3Q19 BGK FP32 64^3 87.9 / 7.9 (8 blocks in all at 64
+    // planes), 128^3 121 / 39.3 (8 planes), 192^3 150 / 124 (28), 320 x 256^2
+    // 410 / 359, 512^3 2343 / 2119, FP16 192^3 127 / 73; D3Q27 KBC FP32 128^3
+    // 139 / 63 (16), 256^3 453 / 432 (128).  256^3 D3Q19 keeps 64 planes (282;
+    // 298 at 32, 300 at 128), 384^3 D3Q27 48.
     tp.cx = knob(K_TB2_PLANES);
     if (tp.cx < 1) {
       tp.cx = 64;
       int per_cu = 0, dev = 0, cus = 0;
       if (hipGetDevice(&dev) == hipSuccess &&
           hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
+          cus > 0 &&
           hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)tb, TB_THREADS, 0) ==
               hipSuccess &&
           per_cu > 0) {
-        const int64_t resident = (int64_t)per_cu * cus;
-        const int64_t tiles64 = (int64_t)tp.nzt * tp.nyt * ((a->n[0] + 63) / 64);
-        // one block per CU (D3Q27): otherwise 48 planes where the rounds of
-        // resident blocks times the planes a block sweeps (cx + 2) come out
-        // lower than for 64.  D3Q27 KBC FP32 384^3: 64 planes make 6.75
-        // rounds, 48 make 9; 35.6k -> 36.2k-37.5k MLUPS (the model ranks the
-        // seven chunk lengths measured there, 32 to 192, in measured order).
-        auto cost = [&](int64_t cx) {
-          const int64_t tiles = (int64_t)tp.nzt * tp.nyt * ((a->n[0] + cx - 1) / cx);
-          return (tiles + resident - 1) / resident * (cx + 2);
-        };
-        if (tiles64 > resident && tiles64 <= 2 * resident) tp.cx = 128;
-        else if (per_cu == 1 && cost(48) < cost(64)) tp.cx = 48;
+        const int64_t column = (int64_t)tp.nzt * tp.nyt;
+        double best = 0;
+        for (int64_t chunks = 1; chunks <= a->n[0]; ++chunks) {
+          const int64_t cx = (a->n[0] + chunks - 1) / chunks;
+          // no chunk from here on sweeps fewer planes than this
+          if (best > 0 && (double)(column * a->n[0]) / cus * (1 + 2.0 / cx) >= best) break;
+          const int64_t share = (column * ((a->n[0] + cx - 1) / cx) + cus - 1) / cus;
+          const double cost = (double)(share * (cx + 2)) * (share < per_cu ? 1.15 : 1.0);
+          if (best == 0 || cost < best) {
+            best = cost;
+            tp.cx = (int)cx;
+          }
+        }
       }
     }
     const int64_t nxt = (a->n[0] + tp.cx - 1) / tp.cx;

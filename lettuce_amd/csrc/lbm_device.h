@@ -109,6 +109,12 @@ template <class T>
 __device__ __forceinline__ T elem(const T* p, uint32_t i) {
   return *elem_ptr(const_cast<T*>(p), i);
 }
+// one store, bypassing the caches (NT) or through them
+template <bool NT, class T>
+__device__ __forceinline__ void put(gptr<T> at, T v) {
+  if constexpr (NT) __builtin_nontemporal_store(v, at);
+  else *at = v;
+}
 // p kept whole in scalar registers: in a loop whose in-plane offsets do not
 // change (the two-step kernel's sweep over planes), the compiler would
 // otherwise hoist base + offset out of the loop as one 64-bit vector
@@ -158,7 +164,7 @@ __device__ __forceinline__ uint32_t sr_bits(uint32_t h, int q) {
 // dec: stored value -> population, enc: population -> stored value;
 // enc_sr: the same with stochastic rounding from 16 random bits r (formats
 // other than BF16 ignore r); ld / st: one element, stores bypassing the
-// caches (streamed output)
+// caches (streamed output) unless NT is false
 struct StF32 {
   using T = float;
   using C = float;
@@ -175,8 +181,9 @@ struct StF32 {
     e[1] = b;
   }
   __device__ static C ld(const T* p, uint32_t i, C) { return elem(p, i); }
+  template <bool NT = true>
   __device__ static void st(T* p, uint32_t i, C v, C) {
-    __builtin_nontemporal_store(v, elem_ptr(p, i));
+    put<NT>(elem_ptr(p, i), v);
   }
 };
 struct StF64 {
@@ -189,8 +196,10 @@ struct StF64 {
   __device__ static T enc(C v, C) { return v; }
   __device__ static T enc_sr(C v, C, uint32_t) { return v; }
   __device__ static C ld(const T* p, uint32_t i, C) { return p[i]; }
+  template <bool NT = true>
   __device__ static void st(T* p, uint32_t i, C v, C) {
-    __builtin_nontemporal_store(v, p + i);
+    if constexpr (NT) __builtin_nontemporal_store(v, p + i);
+    else p[i] = v;
   }
 };
 struct StF16 {
@@ -213,8 +222,9 @@ struct StF16 {
   __device__ static C ld(const T* p, uint32_t i, C sh) {
     return (float)elem(p, i) + sh;
   }
+  template <bool NT = true>
   __device__ static void st(T* p, uint32_t i, C v, C sh) {
-    __builtin_nontemporal_store((_Float16)(v - sh), elem_ptr(p, i));
+    put<NT>(elem_ptr(p, i), (_Float16)(v - sh));
   }
 };
 struct StBF16 {
@@ -247,8 +257,9 @@ struct StBF16 {
   __device__ static C ld(const T* p, uint32_t i, C sh) {
     return bf16_to_f32(elem(p, i)) + sh;
   }
+  template <bool NT = true>
   __device__ static void st(T* p, uint32_t i, C v, C sh) {
-    __builtin_nontemporal_store(f32_to_bf16_rne(v - sh), elem_ptr(p, i));
+    put<NT>(elem_ptr(p, i), f32_to_bf16_rne(v - sh));
   }
 };
 // BF16 storage whose kernels store with stochastic rounding (enc_sr with

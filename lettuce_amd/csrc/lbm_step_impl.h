@@ -43,6 +43,7 @@ struct KParams {
   uint32_t sr_step = 0;   // step index of the launch (its first step)
   uint32_t div2 = 0, div1 = 0;  // FLAT: n2 and n1 as divisors (see fast_div)
   int shift2 = 0, shift1 = 0;
+  int cached = 0;  // stores go through the caches (see fits_cache)
 };
 
 // c / n for c < 2^31 by a multiplication with n's reciprocal, rounded up:
@@ -60,15 +61,14 @@ __host__ __device__ inline uint32_t fast_div(uint32_t c, uint32_t m, int s) {
 // One stored element: to nearest, or with stochastic rounding when the
 // format supports it and the run asks for it (key: sr_step_key of the
 // step, elem: the element's offset, used for the random bits only).
-template <class ST>
+template <class ST, bool NT = true>
 __device__ __forceinline__ void store_elem(const KParams& p, typename ST::T* base, uint32_t i,
                                            typename ST::C v, typename ST::C sh, uint32_t key,
                                            uint32_t elem, int q) {
   if constexpr (ST::stochastic)
-    __builtin_nontemporal_store(ST::enc_sr(v, sh, sr_bits(sr_cell(key, elem), q)),
-                                elem_ptr(base, i));
+    put<NT>(elem_ptr(base, i), ST::enc_sr(v, sh, sr_bits(sr_cell(key, elem), q)));
   else
-    ST::st(base, i, v, sh);
+    ST::template st<NT>(base, i, v, sh);
 }
 
 // Which row (i0, i1) and which run b2 of the row a block takes: rows in
@@ -510,7 +510,7 @@ __device__ __forceinline__ void apply_boundary_op(const KParams& p, const lbm_ce
 // Write the cell's post-collision populations: in place (no post-streaming)
 // or pushed to the neighbours with the streaming rules of the destination.
 // RAW: f holds values to store as they are (no shift subtracted).
-template <class S, class ST, bool MASK, bool PUSH, bool RAW = false, class X>
+template <class S, class ST, bool MASK, bool PUSH, bool RAW = false, bool NT = true, class X>
 __device__ __forceinline__ void store_cell(const KParams& p, int cell, const X (&a0)[3],
                                            const int (&a1)[3], const int (&a2)[3], uint32_t nsm,
                                            uint32_t flags, const typename ST::C (&f)[S::Q]) {
@@ -522,12 +522,12 @@ __device__ __forceinline__ void store_cell(const KParams& p, int cell, const X (
     const uint32_t own = (uint32_t)(a0[1] + a1[1] + a2[1]);
 #pragma unroll
     for (int q = 0; q < S::Q; ++q)
-      store_elem<ST>(p, at_plane(fout + q * p.sq, a0[1]), in_plane(a0[1], a1[1] + a2[1]), f[q],
+      store_elem<ST, NT>(p, at_plane(fout + q * p.sq, a0[1]), in_plane(a0[1], a1[1] + a2[1]), f[q],
                      RAW ? C(0) : shift_of<ST>(S::w[q], p), key, own, q);
   } else if (!MASK) {
 #pragma unroll
     for (int q = 0; q < S::Q; ++q)
-      store_elem<ST>(p, at_plane(fout + q * p.sq, nb_plane<S>(q, +1, a0)),
+      store_elem<ST, NT>(p, at_plane(fout + q * p.sq, nb_plane<S>(q, +1, a0)),
                      in_plane(nb_plane<S>(q, +1, a0), nb_in_plane<S>(q, +1, a1, a2)), f[q],
                      RAW ? C(0) : shift_of<ST>(S::w[q], p), key,
                      (uint32_t)(nb_plane<S>(q, +1, a0) + nb_in_plane<S>(q, +1, a1, a2)), q);
@@ -558,15 +558,13 @@ __device__ __forceinline__ void store_cell(const KParams& p, int cell, const X (
 }
 
 // FLAT: each population's rows are contiguous and its byte offsets fit 32 bits
-template <class S, class ST, int COLL, bool MASK, int MODE, bool FLAT>
-__global__ void __launch_bounds__(256) step_kernel(const KParams p) {
+template <class S, class ST, int COLL, bool MASK, int MODE, bool FLAT, bool NT>
+__device__ __forceinline__ void step_body(const KParams& p, lbm_cell_class* ctl) {
   using C = typename ST::C;
   using T = typename ST::T;
   constexpr bool PULL = (MODE & LBM_PRE_STREAMING) != 0;
   constexpr bool PUSH = (MODE & LBM_POST_STREAMING) != 0;
 
-  // with boundaries, the cell-class table in LDS
-  __shared__ lbm_cell_class ctl[MASK ? 256 : 1];
   if (MASK) {
     stage_classes(p, ctl);
     __syncthreads();
@@ -610,7 +608,24 @@ __global__ void __launch_bounds__(256) step_kernel(const KParams p) {
   const CollParams<C> cp = coll_params<C>(p);
   if (!MASK || op == LBM_OP_COLLIDE) collide<S, C, COLL>(f, cp);
   else apply_boundary_op<S, ST, PULL>(p, ctl, op, flags, cell, i0, i1, i2, f);
-  store_cell<S, ST, MASK, PUSH>(p, cell, a0, a1, a2, nsm, flags, f);
+  store_cell<S, ST, MASK, PUSH, false, NT>(p, cell, a0, a1, a2, nsm, flags, f);
+}
+
+// The whole body stands in both branches of `cached`, so that each schedules
+// its loads, arithmetic and stores as one (a branch around the stores alone
+// cost 2 to 4 %).  Rows of whole wavefronts, most of which the two-step kernels
+// take, always store past the caches.
+template <class S, class ST, int COLL, bool MASK, int MODE, bool FLAT>
+__global__ void __launch_bounds__(256) step_kernel(const KParams p) {
+  // with boundaries, the cell-class table in LDS
+  __shared__ lbm_cell_class ctl[MASK ? 256 : 1];
+  if constexpr (FLAT && MODE == LBM_PRE_STREAMING) {
+    if (p.cached) {
+      step_body<S, ST, COLL, MASK, MODE, FLAT, false>(p, ctl);
+      return;
+    }
+  }
+  step_body<S, ST, COLL, MASK, MODE, FLAT, true>(p, ctl);
 }
 
 

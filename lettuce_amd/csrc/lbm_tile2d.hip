@@ -186,7 +186,8 @@ __global__ void __launch_bounds__(tile2d_max_threads<ST>()) tile2d_kernel(const 
         if (stored) {
           ps.sr_step = p.sr_step + (uint32_t)s;
           const int a1[3] = {0, g1 * p.s1, 0}, a2[3] = {0, g2, 0};
-          store_cell<S, ST, MASK, false>(ps, cell, a0, a1, a2, 0, 0, f);
+          if (p.cached) store_cell<S, ST, MASK, false, false, false>(ps, cell, a0, a1, a2, 0, 0, f);
+          else store_cell<S, ST, MASK, false>(ps, cell, a0, a1, a2, 0, 0, f);
         }
       } else {
         const uint32_t hs = ST::stochastic ? sr_cell(key, (uint32_t)cell) : 0u;
