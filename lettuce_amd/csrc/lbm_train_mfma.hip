@@ -25,6 +25,7 @@
 #include <algorithm>
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 namespace lbm {
 
@@ -96,6 +97,17 @@ __device__ __forceinline__ f32x16 run16(const float* p) {
     v[4 * q + 3] = t.w;
   }
   return v;
+}
+
+__device__ __forceinline__ void run8(const float* p, float (&v)[8]) {
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const float4 t = *(const float4*)(p + 4 * q);
+    v[4 * q] = t.x;
+    v[4 * q + 1] = t.y;
+    v[4 * q + 2] = t.z;
+    v[4 * q + 3] = t.w;
+  }
 }
 
 // the upper half of a changes places with the lower half of b
@@ -279,7 +291,8 @@ __global__ void __launch_bounds__(64 * TM_WAVES, 2)
   float w1a[3];
 #pragma unroll
   for (int j = 0; j < 3; ++j) w1a[j] = w.w1t[2 * j + h][row];
-  f32x16 g2 = {}, g1 = {}, gb2 = {}, g3[3] = {};
+  f32x16 g2 = {}, gb2 = {}, g3[3] = {};
+  f32x4 g1[2] = {};
   float gb3[3] = {};
   const uint32_t cells = (uint32_t)p.ncells;
   const int first = __builtin_amdgcn_readfirstlane(blockIdx.x * TM_WAVES + wave);
@@ -349,7 +362,20 @@ __global__ void __launch_bounds__(64 * TM_WAVES, 2)
         T.dz[unit(i, h)][row] = dz1[i];
       }
       phase();
-      g1 = mfma16(run16(&T.dz[row][16 * h]), run16(&T.x[min(row, 7)][TM_PITCH * blk + 16 * h]), g1);
+      // 7 columns: two products of 16 rows, each quarter of the wave 8 cells
+      {
+        const int quarter = lane >> 4, col = lane & 15;
+        float xs[8];
+        run8(&T.x[min(col, 7)][TM_PITCH * blk + 8 * quarter], xs);
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          float dzs[8];
+          run8(&T.dz[16 * half + col][8 * quarter], dzs);
+#pragma unroll
+          for (int i = 0; i < 8; ++i)
+            g1[half] = __builtin_amdgcn_mfma_f32_16x16x4f32(dzs[i], xs[i], g1[half], 0, 0, 0);
+        }
+      }
 #pragma unroll
       for (int k = 0; k < 6; ++k) {
         phase();
@@ -383,8 +409,6 @@ __global__ void __launch_bounds__(64 * TM_WAVES, 2)
       for (int i = 0; i < 16; ++i) {
         const int u = unit(i, h);
         add(P_W2 + u * HID + row, -LN2 * g2[i]);
-        if (row < 6) add(P_W1 + u * 6 + row, g1[i]);
-        if (row == 6) add(P_B1 + u, g1[i]);
         const float b2 = over_cells(gb2[i]);
         if (row == 0) add(P_B2 + u, b2);
 #pragma unroll
@@ -392,6 +416,13 @@ __global__ void __launch_bounds__(64 * TM_WAVES, 2)
           const float w3 = -LN2 * over_cells(g3[j][i]);
           if (row == 0) add(P_W3 + j * HID + u, w3);
         }
+      }
+      // item i of quarter k of a 16 x 16 product: row 4 k + i, column lane % 16
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int u = 16 * (i / 4) + 4 * (lane >> 4) + i % 4, col = lane & 15;
+        if (col < 6) add(P_W1 + u * 6 + col, g1[i / 4][i % 4]);
+        if (col == 6) add(P_B1 + u, g1[i / 4][i % 4]);
       }
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
