@@ -210,6 +210,8 @@ def copy_ceiling(nbytes, steps, warmup):
 
 # the sources a launch kind's kernel and its launch configuration come from
 KERNEL_SOURCES = {
+    "several-step": ["lbm_tile2d.hip", "lbm_tile2d.h", "lbm_pull2d.h", "lbm_step_impl.h",
+                     "lbm_device.h", "lbm_capi.hip"],
     "two-step": ["lbm_tb2.hip", "lbm_tb2.h", "lbm_step_impl.h", "lbm_device.h", "lbm_capi.hip"],
     "single-step": ["step_d2q9.hip", "step_d3q19.hip", "step_d3q27.hip", "lbm_step_impl.h",
                     "lbm_device.h", "lbm_capi.hip"],
@@ -274,9 +276,10 @@ def write_traffic(name, directory):
     fetch_scale = copy_kib / per_kernel("fetch_copy", "FETCH_SIZE", lambda k: k == copy_name)
     write_scale = copy_kib / per_kernel("write_copy", "WRITE_SIZE", lambda k: k == copy_name)
     rows = _pmc_rows(os.path.join(directory, "fetch_kernel"), "FETCH_SIZE")
-    kind = ("two-step" if any("tb2_kernel" in k for k, _ in rows) else
+    kind = ("several-step" if any("tile2d_kernel" in k for k, _ in rows) else
+            "two-step" if any("tb2_kernel" in k for k, _ in rows) else
             "learned" if any("learned" in k for k, _ in rows) else "single-step")
-    marker = {"two-step": "tb2_kernel", "learned": "learned", "single-step": "step_kernel"}[kind]
+    marker = {"several-step": "tile2d_kernel", "two-step": "tb2_kernel", "learned": "learned", "single-step": "step_kernel"}[kind]
     kname = next(k for k, _ in rows if marker in k)
     fetch = per_kernel("fetch_kernel", "FETCH_SIZE", lambda k: k == kname)
     write = per_kernel("write_kernel", "WRITE_SIZE", lambda k: k == kname)
@@ -466,18 +469,18 @@ def main():
     # populations read + written once per memory pass; the uint8 cell class
     # read once
     bytes_per_cell = 2 * S.q * BYTES[storage] + (1 if sim.cell_classes is not None else 0)
-    pairs, singles = sim._collide_and_stream.plan(args.steps)
-    launches = pairs + singles
+    several, pairs, singles = sim._collide_and_stream.launches(args.steps)
+    launches = several + pairs + singles
     launch_s = gpu_s / launches
     # algorithmic bytes of one launch: every launch reads and writes each
-    # population once, whether it makes one update (single step) or two
-    # (two-step kernel)
+    # population once, whether it makes one update (single step), two
+    # (two-step kernels) or more (several-step kernel)
     algorithmic = bytes_per_cell * cells
     achieved = algorithmic / launch_s / 1e9
-    # the same launches counted per cell update (two per two-step launch):
-    # what single steps would have to move for the same progress
-    single_equiv = (2 * pairs + singles) * bytes_per_cell * cells / launches / launch_s / 1e9
-    kind = "two-step" if pairs else ("learned" if coll == "learned" else "single-step")
+    # the same launches counted per cell update: what single steps would have
+    # to move for the same progress
+    single_equiv = args.steps * bytes_per_cell * cells / launches / launch_s / 1e9
+    kind = "several-step" if several else "two-step" if pairs else ("learned" if coll == "learned" else "single-step")
     traffic, stale = load_traffic(args.workload, kind)
     streaming = "post (collide, then stream)" if args.workload.endswith("_post") \
         else "pre (pull), fused"
@@ -500,7 +503,9 @@ def main():
                    "grid": sim.flow.resolution, "cells": cells,
                    "streaming": streaming, "Re": re, "Ma": ma,
                    "layout": args.layout,
-                   "kernel": ("two-step (two fused steps per launch)" if pairs and not singles
+                   "kernel": (f"{several} several-step + {pairs} two-step + {singles} single-step "
+                              "launches" if several
+                              else "two-step (two fused steps per launch)" if pairs and not singles
                               else "single step" if not pairs
                               else f"{pairs} two-step + {singles} single-step launches")},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1),
