@@ -279,7 +279,8 @@ def write_traffic(name, directory):
     kind = ("several-step" if any("tile2d_kernel" in k for k, _ in rows) else
             "two-step" if any("tb2_kernel" in k for k, _ in rows) else
             "learned" if any("learned" in k for k, _ in rows) else "single-step")
-    marker = {"several-step": "tile2d_kernel", "two-step": "tb2_kernel", "learned": "learned", "single-step": "step_kernel"}[kind]
+    marker = {"several-step": "tile2d_kernel", "two-step": "tb2_kernel", "learned": "learned",
+              "single-step": "step_kernel"}[kind]
     kname = next(k for k, _ in rows if marker in k)
     fetch = per_kernel("fetch_kernel", "FETCH_SIZE", lambda k: k == kname)
     write = per_kernel("write_kernel", "WRITE_SIZE", lambda k: k == kname)

@@ -6,9 +6,8 @@
 // to 250 x 187 cells takes 3 to 4.4 us on MI355X whatever it computes (so:
 // 128^2 BGK FP32 1.5 us, 251 x 187 TRT FP64 2.0 us, a 250 x 125 channel 2.5 us
 // per step, bound by each stage's chain of LDS reads, arithmetic and barrier).
-// Here
-// a block owns a tile of t1 x t2 cells and computes step s (s = 1 .. n) on the
-// tile plus reach * (n - s) cells on each side, so it needs nothing from other
+// Here a block owns a tile of t1 x t2 cells and computes step s (s = 1 .. n) on
+// the tile plus reach * (n - s) cells on each side, so it needs nothing from other
 // blocks until the launch ends; the first step reads the input, the last one
 // writes the output, and the populations between them stay in LDS (two
 // buffers, one barrier per step), rounded to the storage format as a stored
