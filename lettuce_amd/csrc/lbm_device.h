@@ -357,13 +357,11 @@ __device__ __forceinline__ void equilibrium(C rho, const C (&u)[3], C (&feq)[S::
 
 // The same in two operations fewer for each pair, from u scaled by 1.5: the odd
 // part is 2 w rho (e.1.5u) and 4.5 w rho (e.u)^2 that times (e.1.5u).  Rounded
-// differently in the last place, the fused products written out (see
-// collide_kbc).
+// differently in the last place.
 template <class S, class C>
 __device__ __forceinline__ void equilibrium_scaled(C rho, const C (&u)[3], C (&feq)[S::Q]) {
-#pragma clang fp contract(off)
   const C v[3] = {C(1.5) * u[0], C(1.5) * u[1], C(1.5) * u[2]};
-  const C c = C(1) - fma(u[0], v[0], fma(u[1], v[1], u[2] * v[2]));
+  const C c = C(1) - (u[0] * v[0] + u[1] * v[1] + u[2] * v[2]);
 #pragma unroll
   for (int q = 0; q < S::Q; ++q) {
     const int o = S::opp[q];
@@ -375,7 +373,7 @@ __device__ __forceinline__ void equilibrium_scaled(C rho, const C (&u)[3], C (&f
     }
     const C ev = eu_of<S, C>(q, v);
     const C odd = C(2) * wr * ev;
-    const C even = fma(ev, odd, wrc);
+    const C even = wrc + ev * odd;
     feq[q] = even + odd;
     feq[o] = even - odd;
   }
@@ -557,7 +555,6 @@ struct Cube27 {
 // of the size of the deviations), against 171.
 template <class C>
 __device__ __forceinline__ void moments27(const C (&f)[27], C& rho, C (&u)[3], C (&m)[6]) {
-#pragma clang fp contract(off)
   constexpr Cube27 cube;
   C s[3], y1[3], y2[3], z1[3], z2[3], yz[3];  // per x plane
 #pragma unroll
@@ -583,12 +580,12 @@ __device__ __forceinline__ void moments27(const C (&f)[27], C& rho, C (&u)[3], C
   const C ri = recip(rho), third = C(1.0 / 3.0) * drho;
 #pragma unroll
   for (int d = 0; d < 3; ++d) u[d] = j[d] * ri;
-  m[0] = ends - fma(j[0], u[0], third);
-  m[1] = ((y2[2] + y2[0]) + y2[1]) - fma(j[1], u[1], third);
-  m[2] = ((z2[2] + z2[0]) + z2[1]) - fma(j[2], u[2], third);
-  m[3] = fma(-j[0], u[1], y1[2] - y1[0]);
-  m[4] = fma(-j[0], u[2], z1[2] - z1[0]);
-  m[5] = fma(-j[1], u[2], (yz[2] + yz[0]) + yz[1]);
+  m[0] = ends - (third + j[0] * u[0]);
+  m[1] = ((y2[2] + y2[0]) + y2[1]) - (third + j[1] * u[1]);
+  m[2] = ((z2[2] + z2[0]) + z2[1]) - (third + j[2] * u[2]);
+  m[3] = (y1[2] - y1[0]) - j[0] * u[1];
+  m[4] = (z1[2] - z1[0]) - j[0] * u[2];
+  m[5] = ((yz[2] + yz[0]) + yz[1]) - j[1] * u[2];
 }
 
 // KBC (lettuce/ext/_collision/kbc_collision.py:96-160):
@@ -622,10 +619,6 @@ __device__ __forceinline__ void collide_kbc(C (&f)[S::Q], const CollParams<C>& c
     // only: FP64 is bound by memory (no change) and the 2D kernels by
     // latency, where the plain form is the shorter chain (2048 x 512 channel
     // 27.4 against 28.2 us per two steps).
-    // Products are fused with sums only where fma says so: left to the
-    // compiler, this form came out differently in different kernels, and a
-    // slab's faces would not equal the periodic step bit for bit.
-#pragma clang fp contract(off)
     C m[6];
     moments27<C>(f, rho, u, m);
     equilibrium_scaled<S, C>(rho, u, fe);
@@ -633,9 +626,9 @@ __device__ __forceinline__ void collide_kbc(C (&f)[S::Q], const CollParams<C>& c
 #pragma unroll
     for (int q = 0; q < S::Q; ++q) dh[q] = (f[q] - fe[q]) - ds[q];
     const C gamma = kbc_gamma<S, C>(ds, dh, fe, cp);
-    const C keep_s = C(1) - C(2) * cp.beta, keep_h = fma(-gamma, cp.beta, C(1));
+    const C keep_s = C(1) - C(2) * cp.beta, keep_h = C(1) - gamma * cp.beta;
 #pragma unroll
-    for (int q = 0; q < S::Q; ++q) f[q] = fma(keep_h, dh[q], fma(keep_s, ds[q], fe[q]));
+    for (int q = 0; q < S::Q; ++q) f[q] = (fe[q] + keep_s * ds[q]) + keep_h * dh[q];
   } else {
     C df[S::Q];
     moments<S, C>(f, rho, u);
