@@ -355,30 +355,6 @@ __device__ __forceinline__ void equilibrium(C rho, const C (&u)[3], C (&feq)[S::
   }
 }
 
-// The same in two operations fewer for each pair, from u scaled by 1.5: the odd
-// part is 2 w rho (e.1.5u) and 4.5 w rho (e.u)^2 that times (e.1.5u).  Rounded
-// differently in the last place.
-template <class S, class C>
-__device__ __forceinline__ void equilibrium_scaled(C rho, const C (&u)[3], C (&feq)[S::Q]) {
-  const C v[3] = {C(1.5) * u[0], C(1.5) * u[1], C(1.5) * u[2]};
-  const C c = C(1) - (u[0] * v[0] + u[1] * v[1] + u[2] * v[2]);
-#pragma unroll
-  for (int q = 0; q < S::Q; ++q) {
-    const int o = S::opp[q];
-    if (o < q) continue;
-    const C wr = C(S::w[q]) * rho, wrc = wr * c;
-    if (o == q) {
-      feq[q] = wrc;
-      continue;
-    }
-    const C ev = eu_of<S, C>(q, v);
-    const C odd = C(2) * wr * ev;
-    const C even = wrc + ev * odd;
-    feq[q] = even + odd;
-    feq[o] = even - odd;
-  }
-}
-
 // ---------------------------------------------------------------------------
 // Collision operators (the cell's own populations, in place)
 // ---------------------------------------------------------------------------
@@ -475,33 +451,6 @@ __device__ __forceinline__ void collide_trt(C (&f)[S::Q], const CollParams<C>& c
 //      s11,12 = Pxz/4, s13,14 = -Pxz/4, s15,16 = Pxy/4, s17,18 = -Pxy/4,
 //      corners s19..26 = 0                                       (:41-74)
 template <class S, class C>
-__device__ __forceinline__ void kbc_shear_3d(const C (&m)[6], C (&ds)[S::Q]) {
-  const C T = m[0] + m[1] + m[2], Nxz = m[0] - m[2], Nyz = m[1] - m[2];
-  const C sixth = C(1.0 / 6.0);
-  ds[0] = -T;
-  ds[1] = sixth * (C(2) * Nxz - Nyz + T);
-  ds[2] = ds[1];
-  ds[3] = sixth * (C(2) * Nyz - Nxz + T);
-  ds[4] = ds[3];
-  ds[5] = sixth * (-Nxz - Nyz + T);
-  ds[6] = ds[5];
-  ds[7] = C(0.25) * m[5];
-  ds[8] = ds[7];
-  ds[9] = -ds[7];
-  ds[10] = ds[9];
-  ds[11] = C(0.25) * m[4];
-  ds[12] = ds[11];
-  ds[13] = -ds[11];
-  ds[14] = ds[13];
-  ds[15] = C(0.25) * m[3];
-  ds[16] = ds[15];
-  ds[17] = -ds[15];
-  ds[18] = ds[17];
-#pragma unroll
-  for (int q = 19; q < S::Q; ++q) ds[q] = C(0);
-}
-
-template <class S, class C>
 __device__ __forceinline__ void kbc_shear(const C (&df)[S::Q], C (&ds)[S::Q]) {
   if constexpr (S::D == 2) {
     C xx = 0, yy = 0, xy = 0;
@@ -523,69 +472,41 @@ __device__ __forceinline__ void kbc_shear(const C (&df)[S::Q], C (&ds)[S::Q]) {
     ds[7] = ds[5];
     ds[8] = -ds[5];
   } else {
-    C m[6] = {0, 0, 0, 0, 0, 0};  // xx, yy, zz, xy, xz, yz
+    C xx = 0, yy = 0, zz = 0, xy = 0, xz = 0, yz = 0;
 #pragma unroll
     for (int q = 1; q < S::Q; ++q) {
       const int ex = S::e[q][0], ey = S::e[q][1], ez = S::e[q][2];
-      if (ex != 0) m[0] += df[q];
-      if (ey != 0) m[1] += df[q];
-      if (ez != 0) m[2] += df[q];
-      if (ex * ey != 0) m[3] += (ex * ey > 0) ? df[q] : -df[q];
-      if (ex * ez != 0) m[4] += (ex * ez > 0) ? df[q] : -df[q];
-      if (ey * ez != 0) m[5] += (ey * ez > 0) ? df[q] : -df[q];
+      if (ex != 0) xx += df[q];
+      if (ey != 0) yy += df[q];
+      if (ez != 0) zz += df[q];
+      if (ex * ey != 0) xy += (ex * ey > 0) ? df[q] : -df[q];
+      if (ex * ez != 0) xz += (ex * ez > 0) ? df[q] : -df[q];
+      if (ey * ez != 0) yz += (ey * ez > 0) ? df[q] : -df[q];
     }
-    kbc_shear_3d<S, C>(m, ds);
-  }
-}
-
-// D3Q27's population of direction (x - 1, y - 1, z - 1)
-struct Cube27 {
-  int q[3][3][3] = {};
-  constexpr Cube27() {
-    for (int i = 0; i < 27; ++i)
-      q[D3Q27::e[i][0] + 1][D3Q27::e[i][1] + 1][D3Q27::e[i][2] + 1] = i;
-  }
-};
-
-// rho, u and the second-order raw moments (xx, yy, zz, xy, xz, yz) of f - feq
-// for D3Q27.  Those of feq are rho / 3 + rho u_a u_a and rho u_a u_b, so they
-// are taken off the moments of f instead of summing the 18 or 12 differences of
-// each, and f's come from one pass over the lines along z, then y, then x: 84
-// additions with the weights' share taken off in the lines (which leaves sums
-// of the size of the deviations), against 171.
-template <class C>
-__device__ __forceinline__ void moments27(const C (&f)[27], C& rho, C (&u)[3], C (&m)[6]) {
-  constexpr Cube27 cube;
-  C s[3], y1[3], y2[3], z1[3], z2[3], yz[3];  // per x plane
+    const C T = xx + yy + zz, Nxz = xx - zz, Nyz = yy - zz;
+    const C sixth = C(1.0 / 6.0);
+    ds[0] = -T;
+    ds[1] = sixth * (C(2) * Nxz - Nyz + T);
+    ds[2] = ds[1];
+    ds[3] = sixth * (C(2) * Nyz - Nxz + T);
+    ds[4] = ds[3];
+    ds[5] = sixth * (-Nxz - Nyz + T);
+    ds[6] = ds[5];
+    ds[7] = C(0.25) * yz;
+    ds[8] = ds[7];
+    ds[9] = -ds[7];
+    ds[10] = ds[9];
+    ds[11] = C(0.25) * xz;
+    ds[12] = ds[11];
+    ds[13] = -ds[11];
+    ds[14] = ds[13];
+    ds[15] = C(0.25) * xy;
+    ds[16] = ds[15];
+    ds[17] = -ds[15];
+    ds[18] = ds[17];
 #pragma unroll
-  for (int x = 0; x < 3; ++x) {
-    C ls[3], ld[3], lt[3];  // per line: sum, odd and even part of its ends
-#pragma unroll
-    for (int y = 0; y < 3; ++y) {
-      const int q0 = cube.q[x][y][1], qp = cube.q[x][y][2], qm = cube.q[x][y][0];
-      lt[y] = (f[qp] + f[qm]) - C(2 * D3Q27::w[qp]);
-      ld[y] = f[qp] - f[qm];
-      ls[y] = lt[y] + (f[q0] - C(D3Q27::w[q0]));
-    }
-    y2[x] = ls[2] + ls[0];
-    y1[x] = ls[2] - ls[0];
-    s[x] = y2[x] + ls[1];
-    z1[x] = (ld[2] + ld[0]) + ld[1];
-    yz[x] = ld[2] - ld[0];
-    z2[x] = (lt[2] + lt[0]) + lt[1];
+    for (int q = 19; q < S::Q; ++q) ds[q] = C(0);
   }
-  const C ends = s[2] + s[0], drho = ends + s[1];
-  const C j[3] = {s[2] - s[0], (y1[2] + y1[0]) + y1[1], (z1[2] + z1[0]) + z1[1]};
-  rho = C(1) + drho;
-  const C ri = recip(rho), third = C(1.0 / 3.0) * drho;
-#pragma unroll
-  for (int d = 0; d < 3; ++d) u[d] = j[d] * ri;
-  m[0] = ends - (third + j[0] * u[0]);
-  m[1] = ((y2[2] + y2[0]) + y2[1]) - (third + j[1] * u[1]);
-  m[2] = ((z2[2] + z2[0]) + z2[1]) - (third + j[2] * u[2]);
-  m[3] = (y1[2] - y1[0]) - j[0] * u[1];
-  m[4] = (z1[2] - z1[0]) - j[0] * u[2];
-  m[5] = ((yz[2] + yz[0]) + yz[1]) - j[1] * u[2];
 }
 
 // KBC (lettuce/ext/_collision/kbc_collision.py:96-160):
@@ -608,40 +529,17 @@ __device__ __forceinline__ C kbc_gamma(const C (&ds)[S::Q], const C (&dh)[S::Q],
 
 template <class S, class C>
 __device__ __forceinline__ void collide_kbc(C (&f)[S::Q], const CollParams<C>& cp) {
-  C rho, u[3], fe[S::Q], ds[S::Q], dh[S::Q];
-  if constexpr (S::Q == 27 && sizeof(C) == 4) {
-    // Fewer instructions (1325 -> 1145 in the FP32 two-step kernel, which
-    // holds this twice) and f no longer live beside fe and dh, which would
-    // spill there.  Measured in us per step, before / so: FP32 384^3 1556 /
-    // 1532 (two-step, bound by the latency of one block per CU), 256^3
-    // single steps FP16 335 / 318, BF16 345 / 323 (bound by instructions);
-    // the error against FP64 after 20 steps at 384^3 1.0e-6 / 3.4e-7.  FP32
-    // only: FP64 is bound by memory (no change) and the 2D kernels by
-    // latency, where the plain form is the shorter chain (2048 x 512 channel
-    // 27.4 against 28.2 us per two steps).
-    C m[6];
-    moments27<C>(f, rho, u, m);
-    equilibrium_scaled<S, C>(rho, u, fe);
-    kbc_shear_3d<S, C>(m, ds);
+  C rho, u[3], fe[S::Q], df[S::Q], ds[S::Q], dh[S::Q];
+  moments<S, C>(f, rho, u);
+  equilibrium<S, C>(rho, u, fe);
 #pragma unroll
-    for (int q = 0; q < S::Q; ++q) dh[q] = (f[q] - fe[q]) - ds[q];
-    const C gamma = kbc_gamma<S, C>(ds, dh, fe, cp);
-    const C keep_s = C(1) - C(2) * cp.beta, keep_h = C(1) - gamma * cp.beta;
+  for (int q = 0; q < S::Q; ++q) df[q] = f[q] - fe[q];
+  kbc_shear<S, C>(df, ds);
 #pragma unroll
-    for (int q = 0; q < S::Q; ++q) f[q] = (fe[q] + keep_s * ds[q]) + keep_h * dh[q];
-  } else {
-    C df[S::Q];
-    moments<S, C>(f, rho, u);
-    equilibrium<S, C>(rho, u, fe);
+  for (int q = 0; q < S::Q; ++q) dh[q] = df[q] - ds[q];
+  const C gamma = kbc_gamma<S, C>(ds, dh, fe, cp);
 #pragma unroll
-    for (int q = 0; q < S::Q; ++q) df[q] = f[q] - fe[q];
-    kbc_shear<S, C>(df, ds);
-#pragma unroll
-    for (int q = 0; q < S::Q; ++q) dh[q] = df[q] - ds[q];
-    const C gamma = kbc_gamma<S, C>(ds, dh, fe, cp);
-#pragma unroll
-    for (int q = 0; q < S::Q; ++q) f[q] = f[q] - cp.beta * (C(2) * ds[q] + gamma * dh[q]);
-  }
+  for (int q = 0; q < S::Q; ++q) f[q] = f[q] - cp.beta * (C(2) * ds[q] + gamma * dh[q]);
 }
 
 }  // namespace lbm
