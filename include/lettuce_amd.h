@@ -232,7 +232,8 @@ int lbm_run_launches(const lbm_step_args* args, int64_t nsteps, int64_t* launche
  * "multi_step" (the several-step kernel for 2D grids: 0 never, 1 default
  * selection, 2 wherever it applies; "two_step" 0 turns it off too),
  * "multi_step_depth", "multi_step_tile1", "multi_step_tile2" (most steps per
- * launch and the tile's extents, 0 = per grid).  Not synchronised with launches on other threads. */
+ * launch, of which 1 leaves the kernel out, and the tile's extents; 0 = per
+ * grid).  Not synchronised with launches on other threads. */
 int lbm_set_tuning(const char* name, int32_t value);
 
 /* f[q][cell] = feq_q(rho[cell], u[:, cell]) written in the given storage:

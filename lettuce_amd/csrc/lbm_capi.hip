@@ -45,7 +45,7 @@ int launch_learned(const KParams& p, const lbm_learned* l, int stencil, int stor
 //  multi_step         LETTUCE_AMD_MULTI         0 never, 1 the default
 //                                               selection (see tile2d_choice),
 //                                               2 wherever it applies
-//  multi_step_depth   LETTUCE_AMD_MULTI_DEPTH   most steps per launch
+//  multi_step_depth   LETTUCE_AMD_MULTI_DEPTH   most steps per launch (1: none)
 //  multi_step_tile1   LETTUCE_AMD_MULTI_TILE1   tile extents along i1 and i2
 //  multi_step_tile2   LETTUCE_AMD_MULTI_TILE2   (all three: 0 chosen per grid)
 namespace {
@@ -355,6 +355,8 @@ static Tile2dChoice tile2d_choice(const lbm_step_args* a, int64_t nsteps) {
   double best = 0;
   for (const int steps : kSteps) {
     const int k = knob(K_MULTI_DEPTH) > 0 ? (int)std::min<int64_t>(knob(K_MULTI_DEPTH), nsteps) : steps;
+    // (one step per launch leaves the parity's extra launch without a stage)
+    if (k < 2) return ch;
     if (k > nsteps) break;
     for (const auto& t : kTiles) {
       const int t1 = knob(K_MULTI_TILE1) > 0 ? knob(K_MULTI_TILE1) : t[0];
@@ -381,7 +383,7 @@ static Tile2dChoice tile2d_choice(const lbm_step_args* a, int64_t nsteps) {
 
 // Launches of a run of nsteps steps in `stages` stages, at most `most` each: as
 // few as keep the parity of nsteps, so that the result sits where single
-// steps leave it
+// steps leave it (most >= 2 and stages >= 3: never more launches than stages)
 static int64_t tile2d_launches(int64_t nsteps, int64_t stages, int most) {
   const int64_t n = (stages + most - 1) / most;
   return n + ((nsteps - n) & 1);

@@ -126,3 +126,20 @@ def test_default_selection(knobs):
     assert 20 <= several <= 100 and two == 0 and single == 0
     assert launches(ArrayFlow(ctx, _periodic_f0(5, 6), lt.D2Q9()), 10) == (0, 0, 10)
     assert launches(_channel("f32", 2048, 512, "equilibrium", "halfway"), 100) == (0, 50, 0)
+
+
+@pytest.mark.parametrize("strategy", [PRE, POST])
+def test_depth_of_one_step_leaves_the_kernel_out(strategy, knobs):
+    """one step per launch: nothing for the kernel to fuse, and no launch
+    without a stage (a post-order run has one stage more than steps)"""
+    f0 = _periodic_f0(40, 50)
+    for steps in (2, 3, 4, 7):
+        out = []
+        for depth in (1, 0):
+            knobs(multi_step=2 if depth else 0, multi_step_depth=depth, two_step=1 if depth else 0)
+            flow = ArrayFlow(lt.Context("cuda:0", dtype=F64), f0, lt.D2Q9())
+            sim = lt.Simulation(flow, lt.NoCollision(), [], strategy)
+            assert sim._collide_and_stream.launches(steps) == (0, 0, steps)
+            sim(steps)
+            out.append(_bits(flow))
+        assert np.array_equal(out[0], out[1]), steps
