@@ -178,10 +178,15 @@ __device__ __forceinline__ void gather_pull_masked(const KParams& p, const lbm_c
                                                    typename ST::C (&f)[S::Q]) {
   using T = typename ST::T;
   const T* fin = (const T*)p.fin;
+  // the barriers after each load keep the address of the next one from being
+  // computed before this one is issued: a round then holds its results and
+  // one address instead of all of them
   uint32_t cid[S::Q];
 #pragma unroll
-  for (int q = 0; q < S::Q; ++q) cid[q] = p.cls[nb_offset<S>(q, -1, a0, a1, a2)];
-  __builtin_amdgcn_sched_barrier(0);
+  for (int q = 0; q < S::Q; ++q) {
+    cid[q] = elem(p.cls, (uint32_t)nb_offset<S>(q, -1, a0, a1, a2));
+    __builtin_amdgcn_sched_barrier(0);
+  }
   const lbm_cell_class& K = ct[cid[0]];  // e_0 = 0: the cell itself
   const uint32_t nsm = K.no_stream;
   const bool near = (K.flags & (LBM_CLASS_NEAR_SOLID | LBM_CLASS_SOLID)) == LBM_CLASS_NEAR_SOLID;
@@ -189,12 +194,23 @@ __device__ __forceinline__ void gather_pull_masked(const KParams& p, const lbm_c
 #pragma unroll
   for (int q = 1; q < S::Q; ++q) solid |= (ct[cid[q]].flags & LBM_CLASS_SOLID) ? 1u << q : 0u;
   if (!near) solid = 0;
+  // the offsets are found again for the second round: kept from the first,
+  // they would take a register each
+  int b1[3], b2[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    b1[k] = a1[k];
+    b2[k] = a2[k];
+    asm volatile("" : "+v"(b1[k]), "+v"(b2[k]));
+  }
+  __builtin_amdgcn_sched_barrier(0);
   T raw[S::Q];
 #pragma unroll
   for (int q = 0; q < S::Q; ++q) {
     const bool bounce = (solid >> q) & 1u;
-    const int idx = bounce || ((nsm >> q) & 1u) ? cell : nb_offset<S>(q, -1, a0, a1, a2);
+    const int idx = bounce || ((nsm >> q) & 1u) ? cell : nb_offset<S>(q, -1, a0, b1, b2);
     raw[q] = fin[(bounce ? S::opp[q] : q) * p.sq + idx];
+    __builtin_amdgcn_sched_barrier(0);
   }
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -565,6 +581,11 @@ __device__ __forceinline__ void step_body(const KParams& p, lbm_cell_class* ctl)
   constexpr bool PULL = (MODE & LBM_PRE_STREAMING) != 0;
   constexpr bool PUSH = (MODE & LBM_POST_STREAMING) != 0;
 
+  // in scalar registers across the branches of stage_classes: left to the
+  // compiler they come out of those as vector registers, and with them the
+  // row, its neighbours and every population's address
+  const int block = __builtin_amdgcn_readfirstlane(blockIdx.x);
+  const int threads = FLAT ? 256 : __builtin_amdgcn_readfirstlane(blockDim.x);
   if (MASK) {
     stage_classes(p, ctl);
     __syncthreads();
@@ -573,7 +594,7 @@ __device__ __forceinline__ void step_body(const KParams& p, lbm_cell_class* ctl)
   using X = std::conditional_t<FLAT, int, long long>;
   int i0, i1, i2;
   if constexpr (FLAT) {
-    const uint32_t c = blockIdx.x * 256u + threadIdx.x;
+    const uint32_t c = (uint32_t)block * 256u + threadIdx.x;
     if (c >= (uint32_t)p.ncells) return;
     const uint32_t r = fast_div(c, p.div2, p.shift2);
     i2 = (int)(c - r * (uint32_t)p.n2);
@@ -581,8 +602,8 @@ __device__ __forceinline__ void step_body(const KParams& p, lbm_cell_class* ctl)
     i1 = (int)(r - (uint32_t)i0 * (uint32_t)p.n1);
   } else {
     int b2;
-    block_tile(p, blockIdx.x, i0, i1, b2);
-    i2 = b2 * blockDim.x + threadIdx.x;
+    block_tile(p, block, i0, i1, b2);
+    i2 = b2 * threads + threadIdx.x;
     if (i2 >= p.n2) return;
   }
 
@@ -611,12 +632,30 @@ __device__ __forceinline__ void step_body(const KParams& p, lbm_cell_class* ctl)
   store_cell<S, ST, MASK, PUSH, false, NT>(p, cell, a0, a1, a2, nsm, flags, f);
 }
 
+// Wavefronts per SIMD, least and most.  A masked pull step waits for two rounds
+// of loads per cell: its registers leave room for six wavefronts (KBC, which has
+// never had them: five), whatever the rare cells' code would like to hold.
+// us per step with the compiler's own choice of registers for the batched
+// gather of outlet neighbours (D3Q19 83 to 86, D3Q27 103) / now: D3Q27 FP16
+// 256 x 128 x 128 fullway 135 / 109, 128^3 halfway 81 / 68, flat 256 x 100 x 100
+// 97 / 88; D3Q19 FP16 256 x 128 x 128 96 / 81.  FP64 D3Q19, bound by memory,
+// wants no more than four (128^3: 126.9 with five, 124.3).
+template <class S, class ST, int COLL, bool MASK, int MODE>
+constexpr int step_waves(bool most) {
+  if (!MASK || MODE != LBM_PRE_STREAMING) return most ? 8 : 1;
+  if (sizeof(typename ST::C) == 8) return most ? (S::ID == LBM_D3Q19 ? 4 : 8) : 1;
+  return most ? 8 : (S::ID == LBM_D3Q27 && COLL == LBM_COLL_KBC ? 5 : 6);
+}
+
 // The whole body stands in both branches of `cached`, so that each schedules
 // its loads, arithmetic and stores as one (a branch around the stores alone
 // cost 2 to 4 %).  Rows of whole wavefronts, most of which the two-step kernels
 // take, always store past the caches.
 template <class S, class ST, int COLL, bool MASK, int MODE, bool FLAT>
-__global__ void __launch_bounds__(256) step_kernel(const KParams p) {
+__global__ void __launch_bounds__(256)
+    __attribute__((amdgpu_waves_per_eu((step_waves<S, ST, COLL, MASK, MODE>(false)),
+                                       (step_waves<S, ST, COLL, MASK, MODE>(true)))))
+    step_kernel(const KParams p) {
   // with boundaries, the cell-class table in LDS
   __shared__ lbm_cell_class ctl[MASK ? 256 : 1];
   if constexpr (FLAT && MODE == LBM_PRE_STREAMING) {
