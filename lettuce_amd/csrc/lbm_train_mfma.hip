@@ -402,11 +402,21 @@ __global__ void __launch_bounds__(64 * TM_WAVES, 2)
     }
   }
 
-  // the lanes' sums over their cells, then the block's over its waves
+  // the lanes' sums over their cells, all waves at once, then the block's over
+  // its waves, one after the other (with the lanes' sums in that loop, a launch
+  // on 64 cells took 64 us, 28 so)
   auto over_cells = [](float v) {
     for (int o = 16; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     return v;
   };
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    gb2[i] = over_cells(gb2[i]);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) g3[j][i] = over_cells(g3[j][i]);
+  }
+#pragma unroll
+  for (int j = 0; j < 3; ++j) gb3[j] = over_cells(gb3[j]);
   __syncthreads();
   float* red = (float*)turn;
   for (int k = 0; k < TM_WAVES; ++k) {
@@ -416,12 +426,10 @@ __global__ void __launch_bounds__(64 * TM_WAVES, 2)
       for (int i = 0; i < 16; ++i) {
         const int u = unit(i, h);
         add(P_W2 + u * HID + row, -LN2 * g2[i]);
-        const float b2 = over_cells(gb2[i]);
-        if (row == 0) add(P_B2 + u, b2);
+        if (row == 0) {
+          add(P_B2 + u, gb2[i]);
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
-          const float w3 = -LN2 * over_cells(g3[j][i]);
-          if (row == 0) add(P_W3 + j * HID + u, w3);
+          for (int j = 0; j < 3; ++j) add(P_W3 + j * HID + u, -LN2 * g3[j][i]);
         }
       }
       // item i of quarter k of a 16 x 16 product: row 4 k + i, column lane % 16
@@ -432,10 +440,8 @@ __global__ void __launch_bounds__(64 * TM_WAVES, 2)
         if (col == 6) add(P_B1 + u, g1[i / 4][i % 4]);
       }
 #pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const float b3 = over_cells(gb3[j]);
-        if (lane == 0) add(P_B3 + j, b3);
-      }
+      for (int j = 0; j < 3; ++j)
+        if (lane == 0) add(P_B3 + j, gb3[j]);
     }
     __syncthreads();
   }
