@@ -289,98 +289,6 @@ struct Tile2dChoice {
   int t1 = 0, t2 = 0, steps = 0, reach = 1;
 };
 
-// Time of one launch in us, from the waves each CU issues: w[s] wavefronts per
-// tile in step s.  Fitted to 2600 timed launches on MI355X (13 grids of 64^2
-// to 2048^2 cells, 2 to 10 steps, tiles of 4 x 8 to 48 x 96; within 8-14 %
-// each, and the choice it makes within 5 % of the best one timed, 9 % at
-// 2048^2 FP16).  base: an empty launch; sync: one step's latency (loads or LDS,
-// arithmetic, barrier), once per round of resident blocks; issue: one
-// wavefront's step; load: one wavefront's loads of the input.
-struct Tile2dCost {
-  double base, sync, issue, load;
-};
-static double tile2d_cost(const Tile2dCost& c, int n1, int n2, int t1, int t2, int steps, int reach,
-                          int lds, int max_threads, int cu_lds, int cus) {
-  const int tiles = ((n1 + t1 - 1) / t1) * ((n2 + t2 - 1) / t2);
-  int waves = 0, first = 0;
-  for (int s = 0; s < steps; ++s) waves += first = ((t1 + 2 * reach * s) * (t2 + 2 * reach * s) + 63) / 64;
-  const int per_block = std::min(max_threads / 64, first);
-  const int resident = std::max(1, std::min(16, std::min(cu_lds / lds, 2 * (max_threads / 64) / per_block)));
-  const int per_cu = (tiles + cus - 1) / cus;
-  const int rounds = (per_cu + resident - 1) / resident;
-  return c.base + c.sync * (rounds * steps) + c.issue * ((double)waves * per_cu) +
-         c.load * ((double)first * per_cu);
-}
-
-// nsteps: the stages to run (see run_tiles)
-static Tile2dChoice tile2d_choice(const lbm_step_args* a, int64_t nsteps) {
-  Tile2dChoice ch;
-  const int mode = knob(K_MULTI);
-  if (mode == 0 || knob(K_TWO_STEP) == 0 || nsteps <= 2) return ch;
-  if (a->stencil != LBM_D2Q9 || a->streaming != LBM_PRE_STREAMING || a->n[0] != 1) return ch;
-  if (a->collision == LBM_COLL_LEARNED || a->n[1] * a->n[2] > 0x7fffffff) return ch;
-  if (a->stride[3] != 1 || (a->cell_class && a->stride[2] != a->n[2])) return ch;
-  const int bytes = storage_bytes(a->storage);
-  const int64_t last = a->stride[0] * 8 + a->stride[2] * (a->n[1] - 1) + a->n[2] - 1;
-  if (bytes <= 4 ? (last + 1) * bytes >= ((int64_t)1 << 32) : last >= 0x7fffffff) return ch;
-  int dev = 0, max_lds = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
-    return ch;
-  const bool mask = a->cell_class != nullptr, kbc = a->collision == LBM_COLL_KBC;
-  if (mode != 2) {
-    // The row-sweeping two-step kernel computes each cell 1 + 4 / cx times,
-    // a tile more often; with boundaries (twice the overlap) or KBC (twice
-    // the arithmetic) it wins where it applies and its chunks of 8 rows fill
-    // the chip.  Measured in us per step, rows / tiles: 2048 x 512 channel
-    // KBC FP32 13.6 / 16.2, BGK 12.1 / 13.7, KBC FP16 14.1 / 14.9, periodic
-    // KBC 10.8 / 12.4, but BGK 9.3 / 9.2; 1536 x 512 channel KBC 13.9 / 13.1;
-    // 2048 x 256 10.6 / 9.0; 1024 x 1024 BGK FP16 19.5 / 12.1.  Knobs that ask
-    // for the two-step kernel get it.
-    int64_t lds = 0;
-    int nr = 0;
-    const bool rows = two_step_2d(a, &lds, &nr) != nullptr;
-    if (rows && (knob(K_TWO_STEP) == 2 || knob(K_TB2_PLANES) > 0)) return ch;
-    if (rows && (mask || kbc) && a->n[1] >= 8 * (int64_t)cus && a->n[2] >= 512) return ch;
-  }
-  ch.reach = mask ? 2 : 1;
-  static const int kTiles[][2] = {{8, 8},   {8, 16},  {12, 16}, {16, 16}, {8, 32},  {16, 32},
-                                  {24, 32}, {32, 32}, {16, 64}, {24, 48}, {32, 64}, {32, 96}};
-  static const int kSteps[] = {2, 3, 4, 5, 6, 8, 10};
-  const Tile2dCost cost = {mask ? 4.0 : (bytes == 8 ? 4.2 : 2.7),
-                           mask ? (kbc ? 0.64 : 1.1) : (bytes == 8 ? 0.58 : 0.74),
-                           kbc ? 0.085 : (bytes == 8 ? 0.048 : 0.024), 0.15};
-  const int64_t fixed = mask ? tile2d_static_lds_bytes() : 0;
-  double best = 0;
-  for (const int steps : kSteps) {
-    const int k = knob(K_MULTI_DEPTH) > 0 ? (int)std::min<int64_t>(knob(K_MULTI_DEPTH), nsteps) : steps;
-    // (one step per launch leaves the parity's extra launch without a stage)
-    if (k < 2) return ch;
-    if (k > nsteps) break;
-    for (const auto& t : kTiles) {
-      const int t1 = knob(K_MULTI_TILE1) > 0 ? knob(K_MULTI_TILE1) : t[0];
-      const int t2 = knob(K_MULTI_TILE2) > 0 ? knob(K_MULTI_TILE2) : t[1];
-      // one periodic wrap reaches every halo cell
-      const int m = ch.reach * (k - 1);
-      if (t1 + m > a->n[1] || t2 + m > a->n[2]) continue;
-      const int64_t lds = tile2d_lds_bytes(t1, t2, k, ch.reach, bytes, mask) + fixed;
-      if (lds > max_lds) continue;
-      const double us = tile2d_cost(cost, (int)a->n[1], (int)a->n[2], t1, t2, k, ch.reach, (int)lds,
-                                    bytes == 8 ? 512 : 1024, max_lds, cus) / k;
-      if (ch.steps == 0 || us < best) {
-        best = us;
-        ch.t1 = t1;
-        ch.t2 = t2;
-        ch.steps = k;
-      }
-    }
-  }
-  if (ch.steps == 0) return ch;
-  ch.fn = pick_tile2d_kernel(codec_id(a->storage, a->sr_seed), a->collision, mask);
-  return ch;
-}
-
 // Launches of a run of nsteps steps in `stages` stages, at most `most` each: as
 // few as keep the parity of nsteps, so that the result sits where single
 // steps leave it (most >= 2 and stages >= 3: never more launches than stages)
@@ -389,22 +297,15 @@ static int64_t tile2d_launches(int64_t nsteps, int64_t stages, int most) {
   return n + ((nsteps - n) & 1);
 }
 
-// the same for a post-streaming run, which the kernel takes whole; stochastic
-// rounding is keyed to the launches of the split run (see lbm_run)
-static Tile2dChoice tile2d_post_choice(const lbm_step_args* a, int64_t nsteps) {
-  if (a->sr_seed != 0) return Tile2dChoice();
-  lbm_step_args k = *a;
-  k.streaming = LBM_PRE_STREAMING;
-  return tile2d_choice(&k, nsteps + 1);
-}
-
-// Whether both population arrays stay in the device's 256 MB last-level cache
-// from one launch to the next.  The stores then go through the caches; larger
-// arrays are streamed past them, since what a launch writes is gone before the
-// next one reads it.  Measured on MI355X, us per step, past / through: D3Q19
-// FP32 150 x 100 x 90 (205 MB) 40.2 / 34.1, 192 x 96 x 96 (269 MB) 50.5 / 43.9,
-// 128^3 (319 MB) 66.6 / 62.2, 130^3 (334 MB) 66.4 / 67.6, 200^3 (1.2 GB)
-// 214 / 225, D2Q9 2000^2 (288 MB) 51.9 / 49.6.
+// Whether stores go through the caches: where both population arrays take at
+// most `limit` bytes, about the device's 256 MB last-level cache, a launch finds
+// part of what the one before it wrote; larger arrays are streamed past it.  The
+// limits are where the two sides crossed on MI355X, us per step, past / through:
+// single steps with blocks across rows D3Q19 FP32 150 x 100 x 90 (205 MB)
+// 40.2 / 34.1, 192 x 96 x 96 (269 MB) 50.5 / 43.9, 130^3 (334 MB) 66.4 / 67.6,
+// 200^3 (1.2 GB) 214 / 225, D2Q9 2000^2 (288 MB) 51.9 / 49.6; the several-step
+// kernel D2Q9 FP64 1024^2 (151 MB) 17.6 / 17.3, FP32 2000^2 (288 MB) 29.9 / 31.9.
+constexpr int64_t kFlatCached = 300000000, kTilesCached = 200000000;
 static bool fits_cache(const lbm_step_args* a, int64_t limit) {
   return 2 * a->n[0] * a->n[1] * a->n[2] * stencil_q(a->stencil) * storage_bytes(a->storage) <= limit;
 }
@@ -422,6 +323,171 @@ static bool flat_cells(const lbm_step_args* a) {
   const int64_t cells = a->n[0] * a->n[1] * a->n[2];
   return knob(K_FLAT) != 0 && a->n[2] % 64 != 0 && contiguous_cells(a->n, a->stride) &&
          cells < 0x7fffffff && (bytes > 4 || cells * bytes < ((int64_t)1 << 32));
+}
+
+// What a run costs in us, so that 2D grids take the faster kernels: the tiles
+// compute a halo, which pays where a launch or its latency is most of a step,
+// and costs more than it saves where the arithmetic is (large grids, KBC,
+// 16-bit storage).  Fitted to the 7300 launches nearest the best of each grid
+// among 8700 timed on MI355X (14 grids of 32^2 to 3072 x 4096 cells, the tiles
+// and depths below; within 7-12 % each) and to 774 runs without tiles (37
+// grids; within 10 %, single steps 20 %).  us per step, tiles / without:
+// 128^2 BGK FP32 1.6 / 4.5, 1024^2 BGK FP64 17.0 / 31.5, 1500 x 1100 KBC FP16
+// 19.7 / 11.8, 3072 x 4096 KBC FP16 116 / 85, 4096 x 256 KBC FP32 14.0 / 10.7
+// (by rows), 2048 x 512 channel KBC FP32 16.2 / 13.6 (by rows).
+//
+// Launch of the tile kernel.  base: an empty launch; sync: one step's latency
+// (LDS, arithmetic, barrier), once per round of resident blocks; issue: one
+// wavefront's step; stream: a megabyte of the arrays, read or written (FP64 with
+// a class map: 0.03 and 0.05 above the fit, which put its chosen launches 13 %
+// too low).
+struct Tile2dCost {
+  double base, sync, issue, stream;
+};
+// Launch of the row-sweeping two-step kernel.  base as above; iter: one
+// iteration's latency; issue: one wavefront's part in it.
+struct Rows2dCost {
+  double base, iter, issue;
+};
+// by storage (16, 32, 64 bits), class map, KBC
+static const Tile2dCost kTile2dCost[3][2][2] = {
+    {{{5.0, 0.41, 0.066, 0.134}, {5.0, 0.46, 0.109, 0.109}},
+     {{5.7, 0.86, 0.086, 0.145}, {5.6, 0.94, 0.120, 0.136}}},
+    {{{4.8, 0.44, 0.052, 0.140}, {5.1, 0.43, 0.096, 0.104}},
+     {{6.0, 0.87, 0.067, 0.123}, {5.9, 0.94, 0.098, 0.100}}},
+    {{{5.8, 0.28, 0.090, 0.114}, {5.8, 0.45, 0.186, 0.065}},
+     {{5.4, 0.95, 0.125, 0.131}, {5.2, 1.20, 0.203, 0.116}}}};
+static const Rows2dCost kRows2dCost[2][2][2] = {
+    {{{3.5, 0.80, 0.077}, {3.2, 1.01, 0.120}}, {{3.1, 1.80, 0.087}, {6.2, 1.47, 0.126}}},
+    {{{5.5, 0.21, 0.113}, {4.0, 0.75, 0.130}}, {{2.2, 1.84, 0.095}, {5.8, 1.38, 0.134}}}};
+
+static double tile2d_cost(const Tile2dCost& c, const lbm_step_args* a, int t1, int t2, int steps,
+                          int reach, int64_t lds, int max_threads, int64_t cu_lds, int cus) {
+  const int64_t tiles = ((a->n[1] + t1 - 1) / t1) * ((a->n[2] + t2 - 1) / t2);
+  int waves = 0, first = 0;
+  for (int s = 0; s < steps; ++s) waves += first = ((t1 + 2 * reach * s) * (t2 + 2 * reach * s) + 63) / 64;
+  const int per_block = std::min(max_threads / 64, first);
+  const int64_t resident =
+      std::max<int64_t>(1, std::min<int64_t>(16, std::min<int64_t>(cu_lds / lds, 2 * (max_threads / 64) / per_block)));
+  const int64_t per_cu = (tiles + cus - 1) / cus;
+  const int64_t rounds = (per_cu + resident - 1) / resident;
+  const double mb = 2e-6 * D2Q9::Q * storage_bytes(a->storage) * (double)(a->n[1] * a->n[2]);
+  return c.base + c.sync * (double)(rounds * steps) + c.issue * (double)(waves * per_cu) + c.stream * mb;
+}
+
+// one single step: a launch, what a grid adds up to the size that fills the
+// chip, and the arrays at 5.6 TB/s, or 7.4 (16 bits: 8.8) where blocks across
+// rows store through the caches; 16-bit cells with a class map wait longer for
+// their loads
+static double single2d_cost(const lbm_step_args* a) {
+  const bool mask = a->cell_class != nullptr, flat = flat_cells(a);
+  const int bytes = storage_bytes(a->storage);
+  const double mcells = 1e-6 * (double)(a->n[1] * a->n[2]);
+  const double rate = flat && fits_cache(a, kFlatCached) ? (bytes == 2 ? 8.8 : 7.4) : 5.6;
+  double per_cell = 2 * D2Q9::Q * bytes / rate;
+  if (mask && bytes == 2)
+    per_cell = std::max(per_cell, (flat ? 6.6 : 8.7) + (a->collision == LBM_COLL_KBC ? 1.3 : 0.0));
+  const double fill = std::min(1.0, mcells / 0.3);
+  return (mask ? 4.7 : 3.7) + 1.5 * fill * fill + mcells * per_cell;
+}
+
+// nsteps steps without tiles, of which `pull` can go in pairs to the
+// row-sweeping kernel (nr rows per iteration, 0: it does not apply)
+static double other2d_cost(const lbm_step_args* a, int64_t nsteps, int64_t pull, int nr, int64_t lds,
+                           int64_t cu_lds, int cus) {
+  const int64_t pairs = two_step_pairs(nr > 0, pull);
+  double us = (double)(nsteps - 2 * pairs) * single2d_cost(a);
+  if (pairs > 0) {
+    const Rows2dCost& c = kRows2dCost[storage_bytes(a->storage) / 4][a->cell_class != nullptr]
+                                     [a->collision == LBM_COLL_KBC];
+    const int64_t threads = nr * a->n[2];
+    const int64_t resident = std::max<int64_t>(1, std::min(cu_lds / lds, 2048 / threads)) * cus;
+    const int64_t cx = std::max<int64_t>(8, (a->n[1] + resident - 1) / resident);
+    const int64_t blocks = (a->n[1] + cx - 1) / cx, per_cu = (blocks + cus - 1) / cus;
+    const int64_t iters = (cx + 4 + nr - 1) / nr;  // S1 on 4 rows beyond the chunk
+    us += (double)pairs * (c.base + (double)iters * (c.iter + c.issue * (double)(per_cu * threads / 64)));
+  }
+  return us;
+}
+
+// nsteps steps in `stages` stages (see run_tiles)
+static Tile2dChoice tile2d_choice(const lbm_step_args* a, int64_t nsteps, int64_t stages) {
+  Tile2dChoice ch;
+  const int mode = knob(K_MULTI);
+  if (mode == 0 || knob(K_TWO_STEP) == 0 || stages <= 2) return ch;
+  if (a->stencil != LBM_D2Q9 || a->streaming != LBM_PRE_STREAMING || a->n[0] != 1) return ch;
+  if (a->collision == LBM_COLL_LEARNED || a->n[1] * a->n[2] > 0x7fffffff) return ch;
+  if (a->stride[3] != 1 || (a->cell_class && a->stride[2] != a->n[2])) return ch;
+  const int bytes = storage_bytes(a->storage);
+  const int64_t last = a->stride[0] * 8 + a->stride[2] * (a->n[1] - 1) + a->n[2] - 1;
+  if (bytes <= 4 ? (last + 1) * bytes >= ((int64_t)1 << 32) : last >= 0x7fffffff) return ch;
+  int dev = 0, max_lds = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+    return ch;
+  const bool mask = a->cell_class != nullptr, kbc = a->collision == LBM_COLL_KBC;
+  // what the tiles have to beat
+  double best = 0;
+  if (mode != 2) {
+    int64_t lds = 0;
+    int nr = 0;
+    if (two_step_2d(a, &lds, &nr)) {
+      // knobs that ask for the two-step kernel get it
+      if (knob(K_TWO_STEP) == 2 || knob(K_TB2_PLANES) > 0) return ch;
+    } else {
+      nr = 0;
+    }
+    best = other2d_cost(a, nsteps, stages == nsteps ? nsteps : nsteps - 2, nr, lds, max_lds, cus);
+  }
+  ch.reach = mask ? 2 : 1;
+  static const int kTiles[][2] = {{8, 8},   {8, 16},  {12, 16}, {16, 16}, {8, 32},  {16, 32},
+                                  {24, 32}, {32, 32}, {16, 64}, {24, 48}, {32, 64}, {32, 96}};
+  static const int kSteps[] = {2, 3, 4, 5, 6, 8, 10};
+  const Tile2dCost& cost = kTile2dCost[bytes / 4][mask][kbc];
+  const int64_t fixed = mask ? tile2d_static_lds_bytes() : 0;
+  for (const int steps : kSteps) {
+    const int k = knob(K_MULTI_DEPTH) > 0 ? (int)std::min<int64_t>(knob(K_MULTI_DEPTH), stages) : steps;
+    // (one step per launch leaves the parity's extra launch without a stage)
+    if (k < 2) return ch;
+    if (k > stages) break;
+    // the launches as run_tiles makes them: `longer` of them with a stage more
+    const int64_t count = tile2d_launches(nsteps, stages, k), longer = stages % count;
+    const int each = (int)(stages / count);
+    for (const auto& t : kTiles) {
+      const int t1 = knob(K_MULTI_TILE1) > 0 ? knob(K_MULTI_TILE1) : t[0];
+      const int t2 = knob(K_MULTI_TILE2) > 0 ? knob(K_MULTI_TILE2) : t[1];
+      // one periodic wrap reaches every halo cell
+      const int m = ch.reach * (k - 1);
+      if (t1 + m > a->n[1] || t2 + m > a->n[2]) continue;
+      const int64_t lds = tile2d_lds_bytes(t1, t2, k, ch.reach, bytes, mask) + fixed;
+      if (lds > max_lds) continue;
+      auto launches = [&](int64_t number, int stage_count) {
+        return number == 0 ? 0.0
+                           : (double)number * tile2d_cost(cost, a, t1, t2, stage_count, ch.reach, lds,
+                                                          bytes == 8 ? 512 : 1024, max_lds, cus);
+      };
+      const double us = launches(count - longer, each) + launches(longer, each + 1);
+      if (best == 0 || us < best) {
+        best = us;
+        ch.t1 = t1;
+        ch.t2 = t2;
+        ch.steps = k;
+      }
+    }
+  }
+  if (ch.steps == 0) return ch;
+  ch.fn = pick_tile2d_kernel(codec_id(a->storage, a->sr_seed), a->collision, mask);
+  return ch;
+}
+
+// the choice for a post-streaming run, which the kernel takes whole; stochastic
+// rounding is keyed to the launches of the split run (see lbm_run)
+static Tile2dChoice tile2d_post_choice(const lbm_step_args* a, int64_t nsteps) {
+  if (a->sr_seed != 0) return Tile2dChoice();
+  lbm_step_args k = *a;
+  k.streaming = LBM_PRE_STREAMING;
+  return tile2d_choice(&k, nsteps, nsteps + 1);
 }
 
 // Validates the arguments and prepares the single-step kernel (one cell per
@@ -522,7 +588,7 @@ static int prepare_step(const lbm_step_args* a, KParams& p, KernelFn& fn, dim3& 
   p.rho0 = (a->storage == LBM_F16_SHIFTED || a->storage == LBM_BF16_SHIFTED) ? a->rho0_shift : 0.0;
   p.sr_seed = a->sr_seed;
   p.sr_step = a->sr_step;
-  p.cached = fits_cache(a, 300000000);
+  p.cached = fits_cache(a, kFlatCached);
   grid = dim3((unsigned)nb);
   block = dim3(bs);
   return LBM_OK;
@@ -552,8 +618,7 @@ static void run_tiles(const lbm_step_args* a, const KParams& p, const Tile2dChoi
   const int bytes = storage_bytes(a->storage);
   Tile2dParams tp;
   tp.k = p;
-  // (FP64 1024^2, 151 MB: 17.6 / 17.3, FP32 2000^2, 288 MB: 29.9 / 31.9)
-  tp.k.cached = fits_cache(a, 200000000);
+  tp.k.cached = fits_cache(a, kTilesCached);
   tp.t1 = ch.t1;
   tp.t2 = ch.t2;
   tp.reach = ch.reach;
@@ -587,7 +652,7 @@ static void run_tiles(const lbm_step_args* a, const KParams& p, const Tile2dChoi
 static void run_pull_steps(const lbm_step_args* a, const KParams& p, KernelFn fn, dim3 grid,
                            dim3 block, const void* const (&bufs)[2], int64_t& launch,
                            int64_t nsteps, uint32_t& step, hipStream_t s) {
-  const Tile2dChoice ch = tile2d_choice(a, nsteps);
+  const Tile2dChoice ch = tile2d_choice(a, nsteps, nsteps);
   if (ch.fn) {
     run_tiles(a, p, ch, bufs, launch, nsteps, false, step, s);
     return;
@@ -760,7 +825,7 @@ int lbm_run_launches(const lbm_step_args* a, int64_t nsteps, int64_t* launches) 
   const bool whole = split && tile2d_post_choice(a, nsteps).fn;
   const int64_t pull = split && !whole ? nsteps - 2 : nsteps, stages = whole ? nsteps + 1 : pull;
   const Tile2dChoice ch =
-      split || a->streaming == LBM_PRE_STREAMING ? tile2d_choice(&k, stages) : Tile2dChoice();
+      split || a->streaming == LBM_PRE_STREAMING ? tile2d_choice(&k, pull, stages) : Tile2dChoice();
   if (ch.fn) {
     launches[0] = tile2d_launches(pull, stages, ch.steps);
     launches[1] = 0;

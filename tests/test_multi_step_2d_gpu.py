@@ -143,3 +143,20 @@ def test_depth_of_one_step_leaves_the_kernel_out(strategy, knobs):
             sim(steps)
             out.append(_bits(flow))
         assert np.array_equal(out[0], out[1]), steps
+
+
+@pytest.mark.parametrize("storage,nx,ny,coll,order,tiles,rows", [
+    # small, or bound by memory: several steps per launch
+    ("f32", 128, 128, "bgk", POST, True, False), ("f64", 1024, 1024, "bgk", PRE, True, False),
+    ("f32", 700, 701, "kbc", PRE, True, False), ("f16_shifted", 512, 512, "kbc", PRE, True, False),
+    # bound by arithmetic, which the tiles' overlap adds to: without it
+    ("f16_shifted", 1500, 1100, "kbc", POST, False, False),
+    ("f16_shifted", 3072, 4096, "kbc", PRE, False, False),
+    ("f32", 4096, 256, "kbc", PRE, False, True), ("f32", 8192, 128, "kbc", PRE, False, True)])
+def test_tiles_only_where_they_are_faster(storage, nx, ny, coll, order, tiles, rows):
+    flow = lt.TaylorGreenVortex(
+        lt.Context("cuda:0", dtype=F64 if storage == "f64" else F32, storage=storage),
+        [nx, ny], 100, 0.05, lt.D2Q9())
+    sim = lt.Simulation(flow, COLLISIONS[coll](0.6), [], order)
+    several, two, single = sim._collide_and_stream.launches(40)
+    assert (several > 0, two > 0) == (tiles, rows), (several, two, single)
