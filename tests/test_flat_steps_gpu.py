@@ -69,3 +69,8 @@ def test_flat_matches_rows(stencil, res, storage, coll, channel, order, knobs):
     else:
         tol = 5 * TOL[storage] * (50 if coll == "kbc" else 1)
         assert np.abs(out[0][1] - out[1][1]).max() <= tol
+
+
+def test_arrays_past_the_caches(knobs):
+    """two arrays of 302 MB, whose stores bypass the caches, bit for bit"""
+    test_flat_matches_rows("D3Q19", [127, 125, 125], "f32", "none", False, PRE, knobs)

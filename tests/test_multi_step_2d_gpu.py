@@ -160,3 +160,12 @@ def test_tiles_only_where_they_are_faster(storage, nx, ny, coll, order, tiles, r
     sim = lt.Simulation(flow, COLLISIONS[coll](0.6), [], order)
     several, two, single = sim._collide_and_stream.launches(40)
     assert (several > 0, two > 0) == (tiles, rows), (several, two, single)
+
+
+def test_arrays_past_the_caches(knobs):
+    """two arrays of 201 MB, whose stores bypass the caches, bit for bit"""
+    f0 = _periodic_f0(1181, 1181)
+
+    def make():
+        return ArrayFlow(lt.Context("cuda:0", dtype=F64), f0, lt.D2Q9())
+    _compare(make, "f64", "none", PRE, 3, (16, 32), knobs, counts=(4, 5))
