@@ -228,7 +228,8 @@ int lbm_run_launches(const lbm_step_args* args, int64_t nsteps, int64_t* launche
  * "two_step_planes" (x chunk, 0 = per grid), "two_step_barriers" (1 or 2,
  * 0 = per format), "wide_offsets" (1 forces 64-bit plane offsets),
  * "post_split" (0 runs post-streaming with the push kernel only),
- * "flat" (0 runs single steps row by row where rows are no multiple of 64),
+ * "flat" (single steps with blocks across rows, for rows that are no multiple
+ * of 64: 0 never, 1 wherever they apply, 2 default selection),
  * "multi_step" (the several-step kernel for 2D grids: 0 never, 1 default
  * selection, 2 wherever it applies; "two_step" 0 turns it off too),
  * "multi_step_depth", "multi_step_tile1", "multi_step_tile2" (most steps per

@@ -40,8 +40,9 @@ int launch_learned(const KParams& p, const lbm_learned* l, int stencil, int stor
 //                                               offsets (0: chosen per grid)
 //  post_split         LETTUCE_AMD_POST_SPLIT    0 runs post-streaming with the
 //                                               push kernel only (see lbm_run)
-//  flat               LETTUCE_AMD_FLAT          0 runs single steps row by row
-//                                               (see flat_cells)
+//  flat               LETTUCE_AMD_FLAT          single steps across rows: 0 never,
+//                                               1 wherever it applies, 2 the
+//                                               default selection (see flat_cells)
 //  multi_step         LETTUCE_AMD_MULTI         0 never, 1 the default
 //                                               selection (see tile2d_choice),
 //                                               2 wherever it applies
@@ -62,7 +63,7 @@ Knob g_knobs[] = {
     {"two_step_barriers", "LETTUCE_AMD_TB2_BARRIERS", 0, 0, 0},
     {"wide_offsets", "LETTUCE_AMD_WIDE", 0, 0, 0},
     {"post_split", "LETTUCE_AMD_POST_SPLIT", 1, 0, 0},
-    {"flat", "LETTUCE_AMD_FLAT", 1, 0, 0},
+    {"flat", "LETTUCE_AMD_FLAT", 2, 0, 0},
     {"multi_step", "LETTUCE_AMD_MULTI", 1, 0, 0},
     {"multi_step_depth", "LETTUCE_AMD_MULTI_DEPTH", 0, 0, 0},
     {"multi_step_tile1", "LETTUCE_AMD_MULTI_TILE1", 0, 0, 0},
@@ -318,11 +319,24 @@ static bool fits_cache(const lbm_step_args* a, int64_t limit) {
 // (5.1 TB/s), 200^3 298 / 218, 500 x 500 x 33 (TRT) 648 / 223, channel
 // 192 x 96 x 96 64.6 / 61.4; D3Q27 KBC FP32 300^3 1900 / 1063, FP64 200^3
 // 688 / 627, BF16 220 x 220 x 250 460 / 284.
+//
+// Not in FP64 with fewer blocks than CUs (D3Q27 32 x 32 x 48 7.1 / 8.5, KBC
+// 8.2 / 9.8; 50 x 45 x 45, 396 blocks, 13.0 / 9.7), nor where a block takes a whole
+// row, the rows are whole cache lines that fill it well and the arrays are
+// streamed past the caches: D3Q27 FP64 128 x 96 x 224 218 / 232, 192 x 96 x 96
+// 141 / 149, FP32 128 x 96 x 224 115 / 119 (but FP64 96 x 96 x 336, two blocks to a
+// row, 284 / 257, and 100^3, whose rows end inside a line, 91 / 85).
 static bool flat_cells(const lbm_step_args* a) {
   const int bytes = storage_bytes(a->storage);
   const int64_t cells = a->n[0] * a->n[1] * a->n[2];
-  return knob(K_FLAT) != 0 && a->n[2] % 64 != 0 && contiguous_cells(a->n, a->stride) &&
-         cells < 0x7fffffff && (bytes > 4 || cells * bytes < ((int64_t)1 << 32));
+  if (knob(K_FLAT) == 0 || a->n[2] % 64 == 0 || !contiguous_cells(a->n, a->stride) ||
+      cells >= 0x7fffffff || (bytes <= 4 && cells * bytes >= ((int64_t)1 << 32)))
+    return false;
+  if (knob(K_FLAT) == 1) return true;
+  if (bytes == 8 && cells < 256 * 256) return false;
+  const int bs = block_size_for(a->n[2]);
+  return a->n[2] > bs || a->n[2] * bytes % 128 != 0 || fits_cache(a, kFlatCached) ||
+         8 * a->n[2] < (bytes == 8 ? 5 : 7) * bs;
 }
 
 // What a run costs in us, so that 2D grids take the faster kernels: the tiles
