@@ -454,10 +454,12 @@ namespace {
 int tiles_of(int64_t cells) { return (int)((cells + 63) / 64); }
 }  // namespace
 
-// two blocks per CU fit (LDS, registers); a wave sums at least one tile
+// two blocks per CU fit (LDS, registers); a wave sums at least one tile, and at
+// most 32, 2048 cells in one FP32 sum whatever the size, as the partial sums of
+// lbm_learned_grad_reduce
 int train_mfma_blocks(int64_t cells) {
-  const int64_t b = (tiles_of(cells) + TM_WAVES - 1) / TM_WAVES;
-  return (int)(b < 512 ? b : 512);
+  const int64_t rounds = (cells + 64 * TM_WAVES - 1) / (64 * TM_WAVES);  // a tile per wave
+  return (int)(rounds < 512 ? rounds : std::max<int64_t>(512, (rounds + 31) / 32));
 }
 
 void launch_train_forward_mfma(int32_t stencil, const KParams& p, const TrainArgs& t, hipStream_t s) {

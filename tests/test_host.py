@@ -394,3 +394,14 @@ def test_stochastic_rounding_is_a_bf16_context_option():
         lt.Context("cpu", storage="bf16_shifted", rounding="stochastic", rounding_seed=0)
     with pytest.raises(ValueError):
         lt.Context("cpu", rounding="up")
+
+
+@pytest.mark.parametrize("cells", [1, 64, 65, 131073, 32 * 256 * 256, 64 * 256 * 256 + 1, 50_000_000,
+                                   (2 ** 31 - 1) // 9])
+def test_fused_gradient_sums_few_cells_at_a_time(cells):
+    """a wave of the FP32 training kernel keeps one running sum over its
+    cells: at most 2048 of them at any size, as in the record's reduction"""
+    parts, rest = divmod(N.lib().lbm_learned_gradient_workspace(N.F32, cells), 4 * N.LEARNED_PARAMS)
+    assert parts >= 1 and rest == 0
+    waves, tiles = 4 * parts, -(-cells // 64)
+    assert -(-tiles // waves) * 64 <= 2048
