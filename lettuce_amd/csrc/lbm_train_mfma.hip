@@ -40,11 +40,13 @@ namespace {
 
 constexpr int TM_WAVES = 4;
 constexpr int TM_PITCH = 36;  // LDS rows of 32 floats: 16-byte aligned, conflict-free b128 reads
+static_assert(TM_PITCH % 4 == 0 && HID % 4 == 0, "rows read as float4");
 
 // unit held by item r of half h, in groups of four consecutive units
 __device__ constexpr int unit(int r, int h) { return 8 * (r / 4) + 4 * h + r % 4; }
 
-struct WeightsLds {
+// both are read as float4: 16-byte aligned by declaration
+struct alignas(16) WeightsLds {
   float w2[HID][TM_PITCH];   // W2 rows
   float w2t[HID][TM_PITCH];  // W2 columns
   float w1t[6][HID];         // W1 columns
@@ -52,7 +54,7 @@ struct WeightsLds {
   float b1[HID], b2[HID], b3[4];
 };
 // a wave's turned operands; x rows 6 and 7 hold ones and zeros
-struct TurnLds {
+struct alignas(16) TurnLds {
   float a1[HID][TM_PITCH], dz[HID][TM_PITCH], x[8][2 * TM_PITCH];
 };
 
@@ -448,6 +450,7 @@ __global__ void __launch_bounds__(64 * TM_WAVES, 2)
   for (int e = threadIdx.x; e < NPARAM; e += blockDim.x)
     part[(int64_t)blockIdx.x * NPARAM + e] = red[e];
 }
+static_assert(alignof(WeightsLds) == 16 && alignof(TurnLds) == 16, "float4 reads");
 static_assert(sizeof(TurnLds) * TM_WAVES >= NPARAM * sizeof(float), "reduction area");
 
 namespace {
