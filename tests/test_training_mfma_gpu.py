@@ -72,3 +72,36 @@ def test_fused_gradient_is_refused_in_fp64():
     assert N.lib().lbm_learned_gradient_workspace(N.F64, prob.cells) < 0
     with pytest.raises(RuntimeError):
         prob.adjoint_gradient(f, f, False, torch.empty_like(f), theta, theta.clone())
+
+
+@pytest.mark.parametrize("shape", [(5, 241, 251), (67, 65, 63)])
+def test_waves_that_take_several_tiles(shape):
+    """more cells than the kernels' waves hold at once (262144), with a rest:
+    the waves' LDS areas are used again, their sums go on over their tiles.
+    Each block of parameters against its own norm: the rates follow to about
+    1e-4 of their size (see above), and a sum over cells to the same relative
+    error as its terms; three times that."""
+    f = torch.stack([_grid(n=max(shape[1:]), seed=b)[:, :shape[1], :shape[2]]
+                     for b in range(shape[0])], dim=1) if shape[0] == 5 else _populations(shape)
+    theta = _theta(3, out_scale=0.3)
+    lam = torch.rand(f.shape, generator=torch.Generator().manual_seed(7), dtype=F64) - 0.5
+    cfg = lt.TrainConfig(tau=0.57, in_scale=100.0, rate_lo=0.05, rate_hi=1.95)
+    res = {}
+    for dt in (F64, F32):
+        fd, ld = f.to(DEV, dt).contiguous(), lam.to(DEV, dt).contiguous()
+        prob = _Problem(fd, theta.to(DEV, dt), cfg)
+        nxt, mu = torch.full_like(fd, float("nan")), torch.full_like(fd, float("nan"))
+        prob.step(fd, nxt)
+        ws, grad = prob.grad_workspace(), torch.zeros(N.LEARNED_PARAMS, dtype=dt, device=DEV)
+        if prob.fused_gradient:
+            prob.adjoint_gradient(fd, ld, True, mu, ws, grad)
+        else:
+            rec = torch.empty((N.LEARNED_RECORD, prob.cells), dtype=dt, device=DEV)
+            prob.adjoint(fd, ld, True, mu, rec)
+            prob.grad_reduce(rec, ws, grad)
+        blocks = torch.split(grad, [32 * 6, 32, 32 * 32, 32, 3 * 32, 3])
+        res[dt] = [t.double().cpu() for t in (nxt, mu, *blocks)]
+    names = ("state", "adjoint", "W1", "b1", "W2", "b2", "W3", "b3")
+    for name, a, b, tol in zip(names, res[F64], res[F32], [1e-5] + 7 * [3e-4]):
+        err, size = (a - b).norm().item(), a.norm().item()
+        assert err <= tol * size, (name, err, size)
