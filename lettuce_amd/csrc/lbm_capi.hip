@@ -344,8 +344,10 @@ static bool flat_cells(const lbm_step_args* a) {
 // and costs more than it saves where the arithmetic is (large grids, KBC,
 // 16-bit storage).  Fitted to the 7300 launches nearest the best of each grid
 // among 8700 timed on MI355X (14 grids of 32^2 to 3072 x 4096 cells, the tiles
-// and depths below; within 7-12 % each) and to 774 runs without tiles (37
-// grids; within 10 %, single steps 20 %).  us per step, tiles / without:
+// and depths below; within 7-12 % each) and to 906 runs without tiles (40
+// grids; single steps within 20 %, rows 15 %, with a class map 25 %).  Over
+// 2184 runs of 3 to 40 steps the choice is 1 % from the better one in the mean,
+// at worst 16 %.  us per step, tiles / without:
 // 128^2 BGK FP32 1.6 / 4.5, 1024^2 BGK FP64 17.0 / 31.5, 1500 x 1100 KBC FP16
 // 19.7 / 11.8, 3072 x 4096 KBC FP16 116 / 85, 4096 x 256 KBC FP32 14.0 / 10.7
 // (by rows), 2048 x 512 channel KBC FP32 16.2 / 13.6 (by rows).
@@ -383,19 +385,31 @@ static double megabytes2d(const lbm_step_args* a) {
   return 2e-6 * D2Q9::Q * storage_bytes(a->storage) * (double)(a->n[1] * a->n[2]);
 }
 
-static double tile2d_cost(const Tile2dCost& c, const lbm_step_args* a, int t1, int t2, int steps,
-                          int reach, int64_t lds, int max_threads, int64_t cu_lds, int cus) {
-  const int64_t tiles = ((a->n[1] + t1 - 1) / t1) * ((a->n[2] + t2 - 1) / t2);
-  int waves = 0, first = 0;
-  for (int s = 0; s < steps; ++s) waves += first = ((t1 + 2 * reach * s) * (t2 + 2 * reach * s) + 63) / 64;
-  const int per_block = std::min(max_threads / 64, first);
-  const int64_t resident =
-      std::max<int64_t>(1, std::min<int64_t>(16, std::min<int64_t>(cu_lds / lds, 2 * (max_threads / 64) / per_block)));
-  const int64_t per_cu = (tiles + cus - 1) / cus;
-  const int64_t rounds = (per_cu + resident - 1) / resident;
-  return c.base + c.sync * (double)(rounds * steps) + c.issue * (double)(waves * per_cu) +
-         c.stream * megabytes2d(a);
-}
+// A tile's launches of up to `most` steps on one grid; the choice tries many for
+// each run, so the sums over the steps are made once.  No more than 34 steps fit
+// the LDS, with a tile of one cell.
+constexpr int kTile2dSteps = 34;
+struct Tile2dLaunch {
+  int per_cu = 0;  // tiles of the fullest CU
+  // wavefronts of a launch's first step, of all its steps
+  int first[kTile2dSteps + 1], sum[kTile2dSteps + 1];
+  Tile2dLaunch(const lbm_step_args* a, int t1, int t2, int reach, int most, int cus) {
+    const int n1 = (int)a->n[1], n2 = (int)a->n[2];
+    const int tiles = ((n1 + t1 - 1) / t1) * ((n2 + t2 - 1) / t2);
+    per_cu = (tiles + cus - 1) / cus;
+    first[0] = sum[0] = 0;
+    for (int s = 0; s < most; ++s) {
+      first[s + 1] = ((t1 + 2 * reach * s) * (t2 + 2 * reach * s) + 63) / 64;
+      sum[s + 1] = sum[s] + first[s + 1];
+    }
+  }
+  // without the arrays' traffic
+  double us(const Tile2dCost& c, int steps, int by_lds, int max_waves) const {
+    const int resident = std::max(1, std::min(std::min(16, by_lds), 2 * max_waves / std::min(max_waves, first[steps])));
+    const int rounds = (per_cu + resident - 1) / resident;
+    return c.base + c.sync * (double)(rounds * steps) + c.issue * ((double)sum[steps] * per_cu);
+  }
+};
 
 // one single step: a launch, what a grid adds up to the size that fills the
 // chip, and the arrays at 5.6 TB/s, or 7.4 (16 bits: 8.8) where blocks across
@@ -471,28 +485,29 @@ static Tile2dChoice tile2d_choice(const lbm_step_args* a, int64_t nsteps, int64_
   static const int kSteps[] = {2, 3, 4, 5, 6, 8, 10};
   const Tile2dCost& cost = kTile2dCost[bytes / 4][mask][kbc];
   const int64_t fixed = mask ? tile2d_static_lds_bytes() : 0;
-  for (const int steps : kSteps) {
-    const int k = knob(K_MULTI_DEPTH) > 0 ? (int)std::min<int64_t>(knob(K_MULTI_DEPTH), stages) : steps;
-    // (one step per launch leaves the parity's extra launch without a stage)
-    if (k < 2) return ch;
-    if (k > stages) break;
-    // the launches as run_tiles makes them: `longer` of them with a stage more
-    const int64_t count = tile2d_launches(nsteps, stages, k), longer = stages % count;
-    const int each = (int)(stages / count);
-    for (const auto& t : kTiles) {
-      const int t1 = knob(K_MULTI_TILE1) > 0 ? knob(K_MULTI_TILE1) : t[0];
-      const int t2 = knob(K_MULTI_TILE2) > 0 ? knob(K_MULTI_TILE2) : t[1];
+  const int max_waves = bytes == 8 ? 512 / 64 : 1024 / 64;
+  const int most = knob(K_MULTI_DEPTH) > 0 ? std::min(knob(K_MULTI_DEPTH), kTile2dSteps) : 10;
+  const double stream = cost.stream * megabytes2d(a);
+  for (const auto& t : kTiles) {
+    const int t1 = knob(K_MULTI_TILE1) > 0 ? knob(K_MULTI_TILE1) : t[0];
+    const int t2 = knob(K_MULTI_TILE2) > 0 ? knob(K_MULTI_TILE2) : t[1];
+    if (t1 > a->n[1] || t2 > a->n[2] || tile2d_lds_bytes(t1, t2, 2, ch.reach, bytes, mask) > max_lds) continue;
+    const Tile2dLaunch tile(a, t1, t2, ch.reach, most, cus);
+    for (const int steps : kSteps) {
+      const int k = knob(K_MULTI_DEPTH) > 0 ? (int)std::min<int64_t>(knob(K_MULTI_DEPTH), stages) : steps;
+      // (one step per launch leaves the parity's extra launch without a stage)
+      if (k < 2) return ch;
       // one periodic wrap reaches every halo cell
       const int m = ch.reach * (k - 1);
-      if (t1 + m > a->n[1] || t2 + m > a->n[2]) continue;
+      if (k > std::min<int64_t>(stages, most) || t1 + m > a->n[1] || t2 + m > a->n[2]) break;
       const int64_t lds = tile2d_lds_bytes(t1, t2, k, ch.reach, bytes, mask) + fixed;
-      if (lds > max_lds) continue;
-      auto launches = [&](int64_t number, int stage_count) {
-        return number == 0 ? 0.0
-                           : (double)number * tile2d_cost(cost, a, t1, t2, stage_count, ch.reach, lds,
-                                                          bytes == 8 ? 512 : 1024, max_lds, cus);
-      };
-      const double us = launches(count - longer, each) + launches(longer, each + 1);
+      if (lds > max_lds) break;
+      // the launches as run_tiles makes them: `longer` of them with a stage more
+      const int64_t count = tile2d_launches(nsteps, stages, k), longer = stages % count;
+      const int each = (int)(stages / count), by_lds = (int)(max_lds / lds);
+      double us = (double)count * stream;
+      if (count > longer) us += (double)(count - longer) * tile.us(cost, each, by_lds, max_waves);
+      if (longer > 0) us += (double)longer * tile.us(cost, each + 1, by_lds, max_waves);
       if (best == 0 || us < best) {
         best = us;
         ch.t1 = t1;
