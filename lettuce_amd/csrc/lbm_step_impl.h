@@ -649,8 +649,9 @@ constexpr int step_waves(bool most) {
 
 // The whole body stands in both branches of `cached`, so that each schedules
 // its loads, arithmetic and stores as one (a branch around the stores alone
-// cost 2 to 4 %).  Rows of whole wavefronts, most of which the two-step kernels
-// take, always store past the caches.
+// cost 2 to 4 %).  Rows of whole wavefronts always store past the caches: most
+// of those grids run the two-step kernels (the bounded ones, and D3Q27 in FP64
+// and 16 bits, run single steps here at every size; not measured through).
 template <class S, class ST, int COLL, bool MASK, int MODE, bool FLAT>
 __global__ void __launch_bounds__(256)
     __attribute__((amdgpu_waves_per_eu((step_waves<S, ST, COLL, MASK, MODE>(false)),

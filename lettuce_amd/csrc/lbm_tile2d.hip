@@ -5,14 +5,15 @@
 // Small 2D grids are bound by launches, not by work: a single step of 128^2
 // to 250 x 187 cells takes 3 to 4.4 us on MI355X whatever it computes (so:
 // 128^2 BGK FP32 1.5 us, 251 x 187 TRT FP64 2.0 us, a 250 x 125 channel 2.5 us
-// per step, bound by each stage's chain of LDS reads, arithmetic and barrier).
+// per step, bound by each stage's chain of LDS reads, arithmetic and barrier: the
+// VALU is busy 15 to 26 % of a launch).
 // Here a block owns a tile of t1 x t2 cells and computes step s (s = 1 .. n) on
 // the tile plus reach * (n - s) cells on each side, so it needs nothing from other
 // blocks until the launch ends; the first step reads the input, the last one
 // writes the output, and the populations between them stay in LDS (two
 // buffers, one barrier per step), rounded to the storage format as a stored
 // step rounds them.  The overlap is computed more than once, which costs
-// nothing while the chip is mostly idle; the host weighs it (tile2d_plan).
+// nothing while the chip is mostly idle; the host weighs it (tile2d_choice).
 //
 // reach is 1 on periodic grids.  With a class map it is 2: an outlet cell
 // gathers its neighbour x - dir, which itself pulls from one cell further.

@@ -23,10 +23,11 @@
 //
 // Bound by issue: FP32 products on the matrix cores and the VALU's work (64
 // SiLUs and their derivatives, the lattice) take about equal shares and hardly
-// overlap at two waves per SIMD.  D2Q9, 2.1 M cells, before (one thread per cell
-// on the VALU, the record, its reduction) and now: forward 168 / 100 us, adjoint
-// and gradient 1000 / 311 us.  The first layer's gradient on a 32-wide product,
-// mostly padding, took 23 us more.
+// overlap at two waves per SIMD (VALU 42 %, MFMA 39 % of the adjoint's cycles).
+// D2Q9, 2.1 M cells, before (one thread per cell on the VALU, the record, its
+// reduction) and now: forward 168 / 105 us, adjoint and gradient 1000 / 289 us.
+// The first layer's gradient on a 32-wide product, mostly padding, took 23 us
+// more.
 #include "lbm_train_mfma.h"
 
 #include <algorithm>
