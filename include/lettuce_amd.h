@@ -104,8 +104,9 @@ enum lbm_cell_op {
 typedef struct lbm_cell_class {
   uint8_t op;         /* enum lbm_cell_op                                      */
   uint8_t flags;      /* LBM_CLASS_*                                           */
-  int8_t dir[3];      /* OUTLET, ANTI_BOUNCE_BACK: outward normal (i0,i1,i2);
-                         the neighbour velocity is taken at x - dir          */
+  int8_t dir[3];      /* OUTLET, ANTI_BOUNCE_BACK: outward normal (i0,i1,i2),
+                         entries -1, 0 or 1; the neighbour velocity is taken
+                         at x - dir                                          */
   uint8_t pad[3];
   uint32_t no_stream; /* bit q set: population q is not streamed into the cell */
   uint32_t pad2;
